@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64) void raster_backward_kernel(const int* __restri
             sr = splat_b.z;
             sg = splat_b.w;
             sb = splat_c.x;
-            mask = band_mask(mx, my, conic, x0, y0);
+            mask = band_mask<4>(mx, my, conic, x0, y0, 0);
             slot = partial_slot(splat_c, tile_x, tile_y);
         }
 #pragma unroll
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(64) void raster_backward_stored_kernel(const int* _
             sr = splat.b.z;
             sg = splat.b.w;
             sb = splat.c.x;
-            mask = band_mask(mx, my, conic, x0, y0);
+            mask = band_mask<4>(mx, my, conic, x0, y0, 0);
             slot = partial_slot(splat.c, tile_x, tile_y);
         }
 #pragma unroll
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(256) void band_mask_selftest_kernel(const float* sp
         return;
     }
     const float* s = splats + static_cast<int64_t>(i) * 6;
-    masks[i] = band_mask(s[0], s[1], make_float4(s[2], s[3], s[4], s[5]), origins[2 * i], origins[2 * i + 1]);
+    masks[i] = band_mask<4>(s[0], s[1], make_float4(s[2], s[3], s[4], s[5]), origins[2 * i], origins[2 * i + 1], 0);
 }
 
 } // namespace

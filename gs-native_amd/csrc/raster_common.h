@@ -26,6 +26,52 @@ __device__ __forceinline__ int readlane_i(int v, int lane) {
     return __builtin_amdgcn_readlane(v, lane);
 }
 
+// Lane masks as scalars: the lanes whose predicate holds, and back. Combining conditions as 64-bit
+// scalars costs the vector unit nothing beyond the comparisons.
+__device__ __forceinline__ uint64_t lanes_where(bool predicate) {
+    return __builtin_amdgcn_ballot_w64(predicate);
+}
+
+__device__ __forceinline__ bool in_lanes(uint64_t lanes) {
+    return __builtin_amdgcn_inverse_ballot_w64(lanes);
+}
+
+// How many of `lanes` are below this lane.
+__device__ __forceinline__ int lanes_below(uint64_t lanes) {
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(lanes >> 32),
+        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(lanes), 0u));
+}
+
+// Keeps a value in its register: the optimiser can neither recompute nor merge it.
+__device__ __forceinline__ void keep(float& value) {
+    asm volatile("" : "+v"(value));
+}
+
+// Calls f(state, band) for the `Bands` per-band states of a wave. Named states and not an array:
+// an array indexed by the band is moved as a whole vector register on every path.
+template<int Bands, typename State, typename F>
+__device__ __forceinline__ void each_band(State& s0, State& s1, State& s2, State& s3, F f) {
+    f(s0, 0);
+    if constexpr (Bands >= 2) {
+        f(s1, 1);
+    }
+    if constexpr (Bands == 4) {
+        f(s2, 2);
+        f(s3, 3);
+    }
+}
+
+// Alpha of a splat at one pixel, before the 0.99 cap; its exponent (natural, as the reference's
+// `power`) is returned too. across = a dx^2 and along = b dx are shared by a lane's pixels. Forward
+// and backward evaluate exactly these operations, so a replayed pixel blends the same splats.
+__device__ __forceinline__ float splat_alpha(float across, float along, float c, float opacity, float dy,
+    float& power) {
+#pragma clang fp contract(off)
+    constexpr float kLog2e = 1.44269504088896340736f;
+    power = fmaf(fmaf(dy, c * dy, across), -0.5f, -(along * dy));
+    return opacity * __builtin_amdgcn_exp2f(power * kLog2e);
+}
+
 // Bands (bit b = rows [y0 + 4b, y0 + 4b + 3]) of a 16x16 tile at (x0, y0) that the splat's
 // alpha >= 1/255 region can touch. The region is {d : q(d) = d^T Q d <= 2 tau}, tau = ln(255 o),
 // whose half extents are sqrt(2 tau * Sigma_xx) and sqrt(2 tau * Sigma_yy) with Sigma = Q^-1.
@@ -35,30 +81,36 @@ __device__ __forceinline__ int readlane_i(int v, int lane) {
 // Per band, the region's x-range is taken over the band's rows only (the slab's extremes of the
 // ellipse's chords; the ellipse's own extreme point when it lies inside the slab), with the same
 // 2% + 0.5 px margin and never wider than the whole-tile test: a band is kept only if that range
-// meets the tile's 16 columns. Non-finite inputs keep every band.
-__device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x0, int y0) {
+// meets the tile's 16 columns. Non-finite inputs keep every band. The hardware's one-ulp reciprocal,
+// square root and logarithm are far inside the margins (the correctly rounded forms made the mask
+// several times longer).
+// Tests the `Bands` bands from first_band on; bit b stands for band first_band + b.
+template<int Bands>
+__device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x0, int y0, int first_band) {
+    constexpr int kAll = (1 << Bands) - 1;
     float a = conic.x, b = conic.y, c = conic.z, o = conic.w;
     if (!(o >= kAlphaMin)) {
-        return (o == o) ? 0 : 0xf;
+        return (o == o) ? 0 : kAll;
     }
     float det = a * c - b * b;
     if (!(det > 0.0f) || !isfinite(det) || !isfinite(mx) || !isfinite(my)) {
-        return 0xf;
+        return kAll;
     }
-    float tau = logf(255.0f * o) + 0.25f;
+    float tau = __logf(255.0f * o) + 0.25f;
     float two_tau = 2.0f * tau;
-    float sxx = c / det;
-    float syy = a / det;
+    const float inverse_det = __builtin_amdgcn_rcpf(det);
+    float sxx = c * inverse_det;
+    float syy = a * inverse_det;
     float ex2 = two_tau * sxx;
     float ey2 = two_tau * syy;
     float term_bound = (fabsf(a) + fabsf(b)) * ex2 + (fabsf(b) + fabsf(c)) * ey2;
     two_tau += 2e-5f * term_bound;
-    const float ex_raw = sqrtf(two_tau * sxx);
-    const float ey_raw = sqrtf(two_tau * syy);
+    const float ex_raw = __builtin_amdgcn_sqrtf(two_tau * sxx);
+    const float ey_raw = __builtin_amdgcn_sqrtf(two_tau * syy);
     float ext_x = ex_raw * 1.02f + 0.5f;
     float ext_y = ey_raw * 1.02f + 0.5f;
     if (!isfinite(ext_x) || !isfinite(ext_y)) {
-        return 0xf;
+        return kAll;
     }
     const float left = static_cast<float>(x0);
     const float right = static_cast<float>(x0 + 15);
@@ -69,14 +121,14 @@ __device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x
     // dx in [(-b dy - w) / a, (-b dy + w) / a], w = sqrt(2 tau a - det dy^2). Its largest dx is
     // ex_raw at dy = -b ex_raw / c, its smallest -ex_raw at dy = b ex_raw / c; the chord ends
     // are concave / convex in dy, so over a slab without that point the extreme is at an end.
-    const float inverse_a = 1.0f / a;
-    const float dy_of_max = -b * ex_raw / c;
+    const float inverse_a = __builtin_amdgcn_rcpf(a);
+    const float dy_of_max = -b * ex_raw * __builtin_amdgcn_rcpf(c);
     const float two_tau_a = two_tau * a;
     const float x_margin = 0.02f * ex_raw + 0.5f;
     int mask = 0;
 #pragma unroll
-    for (int band = 0; band < 4; ++band) {
-        float lo = static_cast<float>(y0 + 4 * band);
+    for (int band = 0; band < Bands; ++band) {
+        float lo = static_cast<float>(y0 + 4 * (first_band + band));
         float hi = lo + 3.0f;
         if (!(my + ext_y >= lo && my - ext_y <= hi)) {
             continue;
@@ -86,8 +138,8 @@ __device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x
         const float s1 = fminf(my - lo + 0.05f, ey_raw);
         bool keep = true;
         if (s0 <= s1) {
-            const float w0 = sqrtf(fmaxf(two_tau_a - det * s0 * s0, 0.0f));
-            const float w1 = sqrtf(fmaxf(two_tau_a - det * s1 * s1, 0.0f));
+            const float w0 = __builtin_amdgcn_sqrtf(fmaxf(two_tau_a - det * s0 * s0, 0.0f));
+            const float w1 = __builtin_amdgcn_sqrtf(fmaxf(two_tau_a - det * s1 * s1, 0.0f));
             float dx_max = (dy_of_max >= s0 && dy_of_max <= s1) ? ex_raw : fmaxf(-b * s0 + w0, -b * s1 + w1) * inverse_a;
             float dx_min = (-dy_of_max >= s0 && -dy_of_max <= s1) ? -ex_raw
                                                                   : fminf(-b * s0 - w0, -b * s1 - w1) * inverse_a;
