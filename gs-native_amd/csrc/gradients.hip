@@ -369,14 +369,14 @@ __device__ __forceinline__ void reduce_records(const float* __restrict__ partial
         flag1 = record_flags[min(wave_begin + 64 + lane, wave_end - 1)];
     }
     for (int pass = wave_begin; pass < wave_end; pass += kChunks * 64) {
+        // Stamped records (the backward walked them) and, of those, the ones with a partial.
+        const bool stamped0 = pass + lane < wave_end && (flag0 & ~kFlagPartial) == epoch;
+        const bool stamped1 = pass + 64 + lane < wave_end && (flag1 & ~kFlagPartial) == epoch;
         bool reached[kChunks];
-        reached[0] = pass + lane < wave_end && flag0 == epoch;
-        reached[1] = pass + 64 + lane < wave_end && flag1 == epoch;
-        uint64_t ballots[kChunks];
-#pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            ballots[c] = __ballot(reached[c]);
-        }
+        reached[0] = stamped0 && (flag0 & kFlagPartial);
+        reached[1] = stamped1 && (flag1 & kFlagPartial);
+        const uint64_t stamped[kChunks] = {__ballot(stamped0), __ballot(stamped1)};
+        const uint64_t ballots[kChunks] = {__ballot(reached[0]), __ballot(reached[1])};
         const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 a0 = zero, b0 = zero, c0 = zero, a1 = zero, b1 = zero, c1 = zero;
         const int64_t source = 3 * static_cast<int64_t>(pass + lane);
@@ -412,14 +412,14 @@ __device__ __forceinline__ void reduce_records(const float* __restrict__ partial
             const int chunk = pass + c * 64;
             const int low = min(max(begin - chunk, 0), 64);
             const int high = min(max(end - chunk, 0), 64);
-            uint64_t mine = ballots[c];
-            mine &= high >= 64 ? ~0ull : ((1ull << high) - 1);
-            mine &= low >= 64 ? 0ull : ~((1ull << low) - 1);
+            const uint64_t owned = (high >= 64 ? ~0ull : ((1ull << high) - 1)) & (low >= 64 ? 0ull : ~((1ull << low) - 1));
+            uint64_t mine = ballots[c] & owned;
+            const bool wide_owner = __popcll(stamped[c] & owned) >= kWideOwner;
             // Wide owners: each lane takes its own record position if the owner stamped it there,
             // the wave sums the twelve fields and the owner adds the chunk's total. A single new
             // Gaussian can own thousands of records (a screen-filling split), which one lane would
             // otherwise add one LDS round trip at a time while its wave holds the pass open.
-            const uint64_t wide = __ballot(__popcll(mine) >= kWideOwner);
+            const uint64_t wide = __ballot(wide_owner);
             if (wide) {
                 const int own = 3 * (c * 64 + lane);
                 const float4 a = slots[own], b = slots[own + 1], cc = slots[own + 2];
@@ -451,7 +451,7 @@ __device__ __forceinline__ void reduce_records(const float* __restrict__ partial
                         }
                     }
                 }
-                if (__popcll(mine) >= kWideOwner) {
+                if (wide_owner) {
                     mine = 0;
                 }
             }

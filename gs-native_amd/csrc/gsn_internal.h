@@ -86,9 +86,9 @@ struct gsn_context {
     void* slots[kSlotCount] = {};
     size_t slot_bytes[kSlotCount] = {};
     void* pinned = nullptr;  // small pinned host buffer for scalar readbacks
-    // Epoch stamp of the backward's record flags (1..255) and the flag buffer (address and size:
+    // Epoch stamp of the backward's record flags (1..127) and the flag buffer (address and size:
     // a regrown buffer may reuse the address) it was last cleared in: a byte equals the current
-    // epoch only if this step's backward reached that record.
+    // epoch (bit 7 aside) only if this step's backward reached that record.
     uint8_t record_epoch = 0;
     void* record_flags_cleared = nullptr;
     size_t record_flags_cleared_bytes = 0;
@@ -207,6 +207,10 @@ int radix_sort_pairs(gsn_context* context, uint32_t* keys, uint32_t* values, int
 // Floats per (tile, Gaussian) backward partial: dmean2D(2), dSigma2D(3), dlogit, dcolor(3),
 // |dmean2D|(2), pad.
 constexpr int kPartialFloats = 12;
+
+// A record's flag byte: the epoch (1..127) of the step whose backward walked the record, with this
+// bit when some pixel blended it and a partial was written (without it the record's sums are zero).
+constexpr uint8_t kFlagPartial = 0x80;
 
 // Gaussians per workgroup of the per-Gaussian gradient pass.
 constexpr int kGradientGroup = 256;

@@ -155,349 +155,318 @@ __device__ __forceinline__ void store_partial(float* destination, const float4& 
     *reinterpret_cast<float4*>(destination) = value;
 }
 
-__global__ __launch_bounds__(64) void raster_backward_kernel(const int* __restrict__ ids,
+// One pixel of a lane.
+// Recompute form: T is the transmittance in front of the next splat and `walked` the colour of the
+// splats walked so far, summed with the forward's own operations, so that walked - final is exact
+// where the two nearly cancel (walking -final + sums instead, one register less per channel, left
+// the last splats' gradients with the rounding of the whole sum: the share of dmean_x within 1e-5
+// of FP64 on 10,000 Gaussians fell from 0.89 to 0.86). Stored form: T is the transmittance behind
+// the splat being walked and `walked` the colour behind it; `final` is not used. A pixel that is
+// done (outside the image, or terminated) carries T = 0 in the recompute form: every later splat
+// then finds T (1 - alpha) below the termination threshold and blends nothing.
+struct BackwardPixel {
+    float y, T, walked[3], final[3], grad[3];
+    int last;
+};
+
+// Both backward forms. A tile's workgroup has 4 / Bands waves; each owns `Bands` of its four
+// 4-row bands and walks the tile's records in the same batches of 64. A wave's sums over its
+// pixels go to LDS; after the batch the workgroup adds the waves' sums of each record in a fixed
+// order and writes the partials, three lanes a record, so a record's 48 bytes are one piece.
+//
+// What bounds it: VALU issue where there are several waves per SIMD (1080p), the latency of one
+// wave's chain where there are not (a 256x256 image has 256 tiles on 1024 SIMDs), hence the split.
+// The wave-wide sums cost about 30 slots per (record, wave), which is why many tiles keep one wave.
+//
+// Per pair the gradient terms are kept as sums of common * Q d and of its products with Q d; the
+// exact factors (-1 for the mean, 1/2 for the covariance diagonal) are applied to the record's
+// totals. Every record that is walked gets this step's flag, but only those that some pixel of the
+// tile blended get a partial: the others would add exact zeros, 48 bytes written and read each.
+//
+// Stored form (no counterpart in the reference; kept for the memory comparison). The forward stored,
+// per pixel, the final transmittance T_N and the tile-relative index + 1 of the last blended splat.
+// The pass walks each tile's records back to front from the last contributor of any of its pixels,
+// recovering T_k = T_{k+1} / (1 - alpha_k) and the colour behind splat k,
+// B_k = T_N * background + sum_{j > k} c_j alpha_j T_j, so that
+//   dL/dalpha_k = sum_c g_c (T_k c_c - B_c / (1 - alpha_k)),
+// the same quantity as the recompute form's sum_c g_c (prefix_c + T_k c_c - C_c) / (1 - alpha_k).
+template<int Bands, bool Stored>
+__global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const int* __restrict__ ids,
     const int64_t* __restrict__ tile_offsets, const PackedSplat* __restrict__ splats,
     const int* __restrict__ tile_order, Camera cam, const float* __restrict__ image,
-    const float* __restrict__ image_gradients, float* __restrict__ partials, uint8_t* __restrict__ record_flags,
-    uint8_t epoch, int record_count) {
-    __shared__ float s_partial[64 * kPartialFloats];
+    const float* __restrict__ final_transmittance, const int* __restrict__ last_contributor,
+    const float* __restrict__ image_gradients, float bg_r, float bg_g, float bg_b, float* __restrict__ partials,
+    uint8_t* __restrict__ record_flags, uint8_t epoch, int record_count) {
+    constexpr int kWaves = 4 / Bands;
+    // A wave's records of the batch, in order: centre x, y, conic a, b | conic c, opacity, red, green |
+    // blue, 1 - opacity, band mask, lane (the last two as int bits). Every lane reads the same entry (no lane reads). Once walked, an
+    // entry's place takes the record's sums (kPartialFloats is its size too).
+    static_assert(kPartialFloats == 12, "an entry's place holds a record's sums");
+    __shared__ float4 s_list[kWaves][65][3];
+    __shared__ uint64_t s_hits[kWaves];
+    __shared__ uint64_t s_contributed[kWaves];  // by place in the list
+    __shared__ int s_wave[kWaves];  // Stored: a wave's last contributor; else whether it has open pixels
+    __shared__ int s_slot[64];
     const int tile = tile_order[blockIdx.x];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = kWaves == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int first_band = wave * Bands;
     const int tile_x = tile % cam.tile_count_x;
     const int tile_y = tile / cam.tile_count_x;
     const int x0 = tile_x * kTileSize;
     const int y0 = tile_y * kTileSize;
     const int px = x0 + (lane & 15);
-    const int py = y0 + (lane >> 4);
-    const float fx = static_cast<float>(px);
-    // A pixel that is done (outside the image, or terminated) carries T = 0: every later splat
-    // then finds T (1 - alpha) below the termination threshold and blends nothing.
-    float fy[4], T[4], final_color[4][3], grad[4][3], prefix[4][3];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        int y = py + 4 * b;
-        bool inside = px < cam.width && y < cam.height;
-        fy[b] = static_cast<float>(y);
-        T[b] = inside ? 1.0f : 0.0f;
-        int64_t pixel = (static_cast<int64_t>(y) * cam.width + px) * 3;
+    const int py = y0 + 4 * first_band + (lane >> 4);
+    float fx = static_cast<float>(px);
+    keep(fx);
+    BackwardPixel p0, p1, p2, p3;
+    auto each = [&](auto f) { each_band<Bands>(p0, p1, p2, p3, f); };
+    int tile_last = 0;
+    each([&](BackwardPixel& p, int b) {
+        const int y = py + 4 * b;
+        const bool inside = px < cam.width && y < cam.height;
+        const int64_t pixel = static_cast<int64_t>(y) * cam.width + px;
+        p.y = static_cast<float>(y);
+        keep(p.y);
+        p.T = inside ? (Stored ? final_transmittance[pixel] : 1.0f) : (Stored ? 1.0f : 0.0f);
+        p.last = Stored && inside ? last_contributor[pixel] : 0;
+        tile_last = max(tile_last, p.last);
+        const float background[3] = {bg_r, bg_g, bg_b};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            final_color[b][c] = inside ? image[pixel + c] : 0.0f;
-            grad[b][c] = inside ? image_gradients[pixel + c] : 0.0f;
-            prefix[b][c] = 0.0f;
+            p.grad[c] = inside ? image_gradients[pixel * 3 + c] : 0.0f;
+            p.walked[c] = Stored ? p.T * background[c] : 0.0f;
+            p.final[c] = !Stored && inside ? image[pixel * 3 + c] : 0.0f;
         }
-    }
+    });
     const int64_t begin = tile_offsets[tile];
-    const int64_t end = tile_offsets[tile + 1];
+    int64_t end = tile_offsets[tile + 1];
+    if (Stored) {
+        // Largest last contributor over the tile.
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            tile_last = max(tile_last, __shfl_xor(tile_last, offset));
+        }
+        if (kWaves > 1) {
+            if (lane == 0) {
+                s_wave[wave] = tile_last;
+            }
+            __syncthreads();
+            for (int w = 0; w < kWaves; ++w) {
+                tile_last = max(tile_last, s_wave[w]);
+            }
+        }
+        end = min(end, begin + static_cast<int64_t>(tile_last));
+    }
+    // Batch k's records: front to back, or back to front from `end`.
+    const int64_t batches = (end - begin + 63) / 64;
+    auto record_of = [&](int64_t k) {
+        // Of the back-to-front walk the last batch may be the short one: it keeps the lanes of a
+        // full batch, those below `begin` being empty.
+        return Stored ? end - 64 * (k + 1) + lane : begin + 64 * k + lane;
+    };
+    auto has_record = [&](int64_t k) {
+        const int64_t record = record_of(k);
+        return k < batches && record >= begin && record < end;
+    };
     // Software pipeline over record batches: while batch k is processed, the splat records of
     // batch k + 1 and the ids of batch k + 2 are in flight, so the two dependent gathers of a
     // batch (id, then its 48-byte record) are hidden behind a batch of compute.
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float4 current_a = zero, current_b = zero, current_c = zero;
-    if (begin + lane < end) {
-        const PackedSplat* first = splats + ids[begin + lane];
-        current_a = first->a;
-        current_b = first->b;
-        current_c = first->c;
+    PackedSplat following = {zero, zero, zero};
+    if (has_record(0)) {
+        following = splats[ids[record_of(0)]];
     }
-    int following_id = begin + 64 + lane < end ? ids[begin + 64 + lane] : -1;
-    int64_t base = begin;
-    for (; base < end; base += 64) {
-        int active = 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            if (__ballot(T[b] > 0.0f)) {
-                active |= 1 << b;
+    int following_id = has_record(1) ? ids[record_of(1)] : -1;
+    for (int64_t k = 0; k < batches; ++k) {
+        int active = (1 << Bands) - 1;
+        if (!Stored) {
+            active = 0;
+            each([&](BackwardPixel& p, int b) { active |= lanes_where(p.T > 0.0f) ? 1 << b : 0; });
+            if (kWaves == 1) {
+                if (active == 0) {
+                    break;
+                }
+            }
+            else if (lane == 0) {
+                s_wave[wave] = active;
             }
         }
-        if (active == 0) {
-            break;
-        }
-        const float4 splat_a = current_a, splat_b = current_b, splat_c = current_c;
-        if (following_id >= 0) {
-            const PackedSplat* next = splats + following_id;
-            current_a = next->a;
-            current_b = next->b;
-            current_c = next->c;
-        }
-        following_id = base + 128 + lane < end ? ids[base + 128 + lane] : -1;
-        const int64_t record = base + lane;
-        const bool valid = record < end;
-        float mx = 0.0f, my = 0.0f, sr = 0.0f, sg = 0.0f, sb = 0.0f;
-        float4 conic = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        int mask = 0;
-        int64_t slot = 0;
-        if (valid) {
-            mx = splat_a.x;
-            my = splat_a.y;
-            conic = make_float4(splat_a.z, splat_a.w, splat_b.x, splat_b.y);
-            sr = splat_b.z;
-            sg = splat_b.w;
-            sb = splat_c.x;
-            mask = band_mask<4>(mx, my, conic, x0, y0, 0);
-            slot = partial_slot(splat_c, tile_x, tile_y);
-        }
+        if (kWaves > 1) {
+            // Also ends the reads of the previous batch's sums.
+            __syncthreads();
+            if (!Stored) {
+                int any = 0;
 #pragma unroll
-        for (int k = 0; k < kPartialFloats; ++k) {
-            s_partial[lane * kPartialFloats + k] = 0.0f;
+                for (int w = 0; w < kWaves; ++w) {
+                    any |= s_wave[w];
+                }
+                if (any == 0) {
+                    break;
+                }
+            }
         }
-        __syncthreads();
-        uint64_t pending = __ballot((mask & active) != 0);
-        while (pending) {
-            const int j = __builtin_ctzll(pending);
-            pending &= pending - 1;
-            const int smask = readlane_i(mask, j) & active;
-            const float sx = readlane_f(mx, j);
-            const float sy = readlane_f(my, j);
-            const float ca = readlane_f(conic.x, j);
-            const float cbv = readlane_f(conic.y, j);
-            const float cc = readlane_f(conic.z, j);
-            const float op = readlane_f(conic.w, j);
-            const float col[3] = {readlane_f(sr, j), readlane_f(sg, j), readlane_f(sb, j)};
-            const float dx = sx - fx;
+        const bool valid = has_record(k);
+        const float4 conic = make_float4(following.a.z, following.a.w, following.b.x, following.b.y);
+        int mask = 0;
+        if (valid) {
+            mask = band_mask<Bands>(following.a.x, following.a.y, conic, x0, y0, first_band) & active;
+        }
+        const uint64_t hits = lanes_where(mask != 0);
+        if (mask != 0) {
+            const int place = lanes_below(hits);
+            s_list[wave][place][0] = make_float4(following.a.x, following.a.y, conic.x, conic.y);
+            s_list[wave][place][1] = make_float4(conic.z, conic.w, following.b.z, following.b.w);
+            s_list[wave][place][2] =
+                make_float4(following.c.x, 1.0f - conic.w, __int_as_float(mask), __int_as_float(lane));
+        }
+        if (wave == 0) {
+            s_slot[lane] = valid ? static_cast<int>(partial_slot(following.c, tile_x, tile_y)) : -1;
+        }
+        if (following_id >= 0) {
+            following = splats[following_id];
+        }
+        following_id = has_record(k + 2) ? ids[record_of(k + 2)] : -1;
+        const int tile_index = static_cast<int>(record_of(k) - lane - begin);  // of lane 0's record
+        uint64_t contributed = 0;
+        const int entries = __popcll(hits);
+        auto place_of = [&](int step) { return Stored ? entries - 1 - step : step; };
+        __builtin_amdgcn_wave_barrier();
+        float4 next_a = s_list[wave][max(place_of(0), 0)][0];
+        float4 next_b = s_list[wave][max(place_of(0), 0)][1];
+        float4 next_c = s_list[wave][max(place_of(0), 0)][2];
+        for (int step = 0; step < entries; ++step) {
+            const int place = place_of(step);
+            const float4 a = next_a, b4 = next_b, c4 = next_c;
+            const int ahead = Stored ? max(place - 1, 0) : place + 1;
+            next_a = s_list[wave][ahead][0];
+            next_b = s_list[wave][ahead][1];
+            next_c = s_list[wave][ahead][2];
+            const int smask = Bands == 1 ? 1 : __builtin_amdgcn_readfirstlane(__float_as_int(c4.z));
+            const float ca = a.z, cbv = a.w, cc = b4.x, op = b4.y;
+            const float dx = a.x - fx;
+            const float along = cbv * dx;
+            const float ca_dx = ca * dx;
+            const float across = dx * ca_dx;
             float acc[12];
 #pragma unroll
-            for (int k = 0; k < 12; ++k) {
-                acc[k] = 0.0f;
+            for (int f = 0; f < 12; ++f) {
+                acc[f] = 0.0f;
                 // Opaque to the optimiser: otherwise it folds the zero into the first band's
                 // update and rebuilds twelve zeros on every path that skips a band.
-                asm volatile("" : "+v"(acc[k]));
+                if (Bands > 1) {
+                    keep(acc[f]);
+                }
             }
-            bool contributed = false;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
+            uint64_t blended = 0;
+            each([&](BackwardPixel& p, int b) {
+#pragma clang fp contract(off)
                 if (smask & (1 << b)) {
-                    float dy = sy - fy[b];
-                    float power = -0.5f * (ca * dx * dx + cc * dy * dy) - cbv * dx * dy;
-                    float raw_alpha = op * __expf(power);
-                    float alpha = fminf(kAlphaMax, raw_alpha);
-                    bool take = !(power > 0.0f) && alpha >= kAlphaMin;
-                    float next = T[b] * (1.0f - alpha);
-                    bool finish = take && next < kTransmittanceMin;
-                    bool blend = take && !finish;
+                    const float dy = a.y - p.y;
+                    float power;
+                    const float raw_alpha = splat_alpha(across, along, cc, op, dy, power);
+                    const float alpha = fminf(kAlphaMax, raw_alpha);
+                    const float through = 1.0f - alpha;
+                    const uint64_t take = lanes_where(!(power > 0.0f)) & lanes_where(alpha >= kAlphaMin);
+                    const float next = p.T * through;
+                    const uint64_t open = Stored ? lanes_where(tile_index + __float_as_int(c4.w) < p.last)
+                                                 : lanes_where(next >= kTransmittanceMin);
+                    const uint64_t blend = take & open;
                     // Uniform branch on "some lane blends"; inside, lanes that do not blend add
                     // exact zeros (selects, not divergent ifs), which keeps the accumulators in
                     // place instead of merging per-lane control paths.
-                    if (__ballot(blend)) {
-                        contributed = true;
-                        float weight = blend ? alpha * T[b] : 0.0f;
-                        float inv = __builtin_amdgcn_rcpf(1.0f - alpha);
-                        float alpha_gradient = 0.0f;
+                    if (blend) {
+                        blended |= blend;
+                        const float inv = __builtin_amdgcn_rcpf(through);
+                        const float before = Stored ? p.T * inv : p.T;
+                        const float weight = in_lanes(blend) ? alpha * before : 0.0f;
+                        const float colour[3] = {b4.z, b4.w, c4.x};
+                        float sum = 0.0f;
 #pragma unroll
                         for (int c = 0; c < 3; ++c) {
-                            alpha_gradient += grad[b][c] * (prefix[b][c] + T[b] * col[c] - final_color[b][c]) * inv;
-                            acc[6 + c] += weight * grad[b][c];
+                            const float difference = Stored ? fmaf(before, colour[c], -p.walked[c] * inv)
+                                                            : fmaf(colour[c], before, p.walked[c]) - p.final[c];
+                            sum = Stored ? fmaf(p.grad[c], difference, sum) : fmaf(inv, p.grad[c] * difference, sum);
+                            acc[6 + c] = fmaf(weight, p.grad[c], acc[6 + c]);
+                            p.walked[c] = fmaf(colour[c], weight, p.walked[c]);
                         }
-                        float common = blend && raw_alpha < kAlphaMax ? alpha_gradient * raw_alpha : 0.0f;
-                        float qx = ca * dx + cbv * dy;
-                        float qy = cbv * dx + cc * dy;
-                        float gx = -common * qx;
-                        float gy = -common * qy;
-                        acc[0] += gx;
-                        acc[1] += gy;
-                        acc[2] += 0.5f * common * qx * qx;
-                        acc[3] += common * qx * qy;
-                        acc[4] += 0.5f * common * qy * qy;
-                        acc[5] += common * (1.0f - op);
+                        const uint64_t uncapped = blend & lanes_where(raw_alpha < kAlphaMax);
+                        const float common = in_lanes(uncapped) ? raw_alpha * sum : 0.0f;
+                        const float qx = fmaf(cbv, dy, ca_dx);
+                        const float qy = along + cc * dy;
+                        const float gx = common * qx;
+                        const float gy = common * qy;
+                        acc[0] = fmaf(qx, common, acc[0]);
+                        acc[1] = fmaf(qy, common, acc[1]);
+                        acc[2] = fmaf(qx, gx, acc[2]);
+                        acc[3] = fmaf(qy, gx, acc[3]);
+                        acc[4] = fmaf(qy, gy, acc[4]);
+                        acc[5] = fmaf(c4.y, common, acc[5]);
                         acc[9] += fabsf(gx);
                         acc[10] += fabsf(gy);
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            prefix[b][c] += col[c] * weight;
-                        }
-                        T[b] = blend ? next : T[b];
+                        p.T = in_lanes(blend) ? (Stored ? before : next) : p.T;
                     }
-                    T[b] = finish ? 0.0f : T[b];
+                    if (!Stored && (take & ~open)) {
+                        keep(p.T);
+                        p.T = in_lanes(take & ~open) ? 0.0f : p.T;
+                    }
                 }
-            }
-            if (contributed) {
+            });
+            if (blended) {
+                contributed |= 1ull << place;
                 float sums[3];
                 wave_sum12(acc, sums);
                 if ((lane & 15) == 0) {
-                    int row = lane >> 4;
+                    float* destination = reinterpret_cast<float*>(s_list[wave][place]) + 3 * (lane >> 4);
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        s_partial[j * kPartialFloats + 3 * row + k] = sums[k];
+                    for (int f = 0; f < 3; ++f) {
+                        destination[f] = sums[f];
                     }
                 }
             }
         }
-        __syncthreads();
-        if (valid && slot >= 0 && slot < record_count) {
-            const float4* source = reinterpret_cast<const float4*>(s_partial + lane * kPartialFloats);
-            float* destination = partials + slot * kPartialFloats;
-            store_partial(destination, source[0]);
-            store_partial(destination + 4, source[1]);
-            store_partial(destination + 8, source[2]);
-            record_flags[slot] = epoch;
+        if (kWaves > 1 && lane == 0) {
+            s_hits[wave] = hits;
+            s_contributed[wave] = contributed;
         }
         __syncthreads();
-    }
-    // Records after every pixel of the tile terminated contribute nothing; they get neither a
-    // partial nor this step's flag.
-}
-
-// Stored-state variant (no counterpart in the reference; kept for the memory comparison with the
-// recompute form above). The forward stored, per pixel, the final transmittance T_N and the
-// tile-relative index + 1 of the last blended splat. The pass walks each tile's records back to
-// front from the last contributor of any of its pixels, recovering T_k = T_{k+1} / (1 - alpha_k)
-// and the colour behind splat k, B_k = T_N * background + sum_{j > k} c_j alpha_j T_j, so that
-//   dL/dalpha_k = sum_c g_c (T_k c_c - B_c / (1 - alpha_k)),
-// the same quantity as the recompute form's sum_c g_c (prefix_c + T_k c_c - C_c) / (1 - alpha_k).
-// Partials go to the same per-record slots.
-__global__ __launch_bounds__(64) void raster_backward_stored_kernel(const int* __restrict__ ids,
-    const int64_t* __restrict__ tile_offsets, const PackedSplat* __restrict__ splats,
-    const int* __restrict__ tile_order, Camera cam, const float* __restrict__ final_transmittance,
-    const int* __restrict__ last_contributor, const float* __restrict__ image_gradients, float bg_r, float bg_g,
-    float bg_b, float* __restrict__ partials, uint8_t* __restrict__ record_flags, uint8_t epoch, int record_count) {
-    __shared__ float s_partial[64 * kPartialFloats];
-    const int tile = tile_order[blockIdx.x];
-    const int lane = threadIdx.x;
-    const int tile_x = tile % cam.tile_count_x;
-    const int tile_y = tile / cam.tile_count_x;
-    const int x0 = tile_x * kTileSize;
-    const int y0 = tile_y * kTileSize;
-    const int px = x0 + (lane & 15);
-    const int py = y0 + (lane >> 4);
-    const float fx = static_cast<float>(px);
-    const float background[3] = {bg_r, bg_g, bg_b};
-    float fy[4], T[4], behind[4][3], grad[4][3];
-    int last[4];
-    int tile_last = 0;
+        // 64 records x three 16-byte pieces; consecutive lanes write a record's consecutive pieces.
+        for (int item = threadIdx.x; item < 64 * 3; item += 64 * kWaves) {
+            const int record = item / 3;
+            const int piece = item - 3 * record;
+            float4 sum = zero;
+            bool any = false;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        int y = py + 4 * b;
-        bool inside = px < cam.width && y < cam.height;
-        fy[b] = static_cast<float>(y);
-        int64_t pixel = static_cast<int64_t>(y) * cam.width + px;
-        T[b] = inside ? final_transmittance[pixel] : 1.0f;
-        last[b] = inside ? last_contributor[pixel] : 0;
-        tile_last = max(tile_last, last[b]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            grad[b][c] = inside ? image_gradients[pixel * 3 + c] : 0.0f;
-            behind[b][c] = T[b] * background[c];
-        }
-    }
-    // Largest last contributor over the tile (wave maximum through LDS-free lane reads).
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
-        tile_last = max(tile_last, __shfl_xor(tile_last, offset));
-    }
-    const int64_t begin = tile_offsets[tile];
-    const int64_t end = tile_offsets[tile + 1];
-    const int64_t stop = min(end, begin + static_cast<int64_t>(tile_last));
-    for (int64_t top = stop; top > begin; top -= 64) {
-        const int64_t base = max(begin, top - 64);
-        const int64_t record = base + lane;
-        const bool valid = record < top;
-        float mx = 0.0f, my = 0.0f, sr = 0.0f, sg = 0.0f, sb = 0.0f;
-        float4 conic = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        int mask = 0;
-        int64_t slot = 0;
-        if (valid) {
-            const PackedSplat splat = splats[ids[record]];
-            mx = splat.a.x;
-            my = splat.a.y;
-            conic = make_float4(splat.a.z, splat.a.w, splat.b.x, splat.b.y);
-            sr = splat.b.z;
-            sg = splat.b.w;
-            sb = splat.c.x;
-            mask = band_mask<4>(mx, my, conic, x0, y0, 0);
-            slot = partial_slot(splat.c, tile_x, tile_y);
-        }
-#pragma unroll
-        for (int k = 0; k < kPartialFloats; ++k) {
-            s_partial[lane * kPartialFloats + k] = 0.0f;
-        }
-        __syncthreads();
-        uint64_t pending = __ballot(mask != 0);
-        while (pending) {
-            const int j = 63 - __builtin_clzll(pending);
-            pending &= ~(1ull << j);
-            const int position = static_cast<int>(base - begin) + j;  // tile-relative record index
-            const int smask = readlane_i(mask, j);
-            const float sx = readlane_f(mx, j);
-            const float sy = readlane_f(my, j);
-            const float ca = readlane_f(conic.x, j);
-            const float cbv = readlane_f(conic.y, j);
-            const float cc = readlane_f(conic.z, j);
-            const float op = readlane_f(conic.w, j);
-            const float col[3] = {readlane_f(sr, j), readlane_f(sg, j), readlane_f(sb, j)};
-            const float dx = sx - fx;
-            float acc[12];
-#pragma unroll
-            for (int k = 0; k < 12; ++k) {
-                acc[k] = 0.0f;
-            }
-            bool contributed = false;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if (smask & (1 << b)) {
-                    float dy = sy - fy[b];
-                    float power = -0.5f * (ca * dx * dx + cc * dy * dy) - cbv * dx * dy;
-                    float raw_alpha = op * __expf(power);
-                    float alpha = fminf(kAlphaMax, raw_alpha);
-                    bool blend = position < last[b] && !(power > 0.0f) && alpha >= kAlphaMin;
-                    if (blend) {
-                        contributed = true;
-                        float inv = __builtin_amdgcn_rcpf(1.0f - alpha);
-                        float before = T[b] * inv;  // T_k, transmittance in front of this splat
-                        float weight = alpha * before;
-                        float alpha_gradient = 0.0f;
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            alpha_gradient += grad[b][c] * (before * col[c] - behind[b][c] * inv);
-                            acc[6 + c] += weight * grad[b][c];
-                        }
-                        if (raw_alpha < kAlphaMax) {
-                            float common = alpha_gradient * raw_alpha;
-                            float qx = ca * dx + cbv * dy;
-                            float qy = cbv * dx + cc * dy;
-                            float gx = -common * qx;
-                            float gy = -common * qy;
-                            acc[0] += gx;
-                            acc[1] += gy;
-                            acc[2] += 0.5f * common * qx * qx;
-                            acc[3] += common * qx * qy;
-                            acc[4] += 0.5f * common * qy * qy;
-                            acc[5] += common * (1.0f - op);
-                            acc[9] += fabsf(gx);
-                            acc[10] += fabsf(gy);
-                        }
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            behind[b][c] += col[c] * weight;
-                        }
-                        T[b] = before;
-                    }
+            for (int w = 0; w < kWaves; ++w) {
+                const uint64_t listed = kWaves == 1 ? hits : s_hits[w];
+                const uint64_t mine = kWaves == 1 ? contributed : s_contributed[w];
+                const int place = __popcll(listed & ((1ull << record) - 1));
+                if (((listed >> record) & 1) && ((mine >> place) & 1)) {
+                    const float4 v = s_list[w][place][piece];
+                    sum = make_float4(sum.x + v.x, sum.y + v.y, sum.z + v.z, sum.w + v.w);
+                    any = true;
                 }
             }
-            if (__ballot(contributed)) {
-                float sums[3];
-                wave_sum12(acc, sums);
-                if ((lane & 15) == 0) {
-                    int row = lane >> 4;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        s_partial[j * kPartialFloats + 3 * row + k] = sums[k];
-                    }
+            const int slot = s_slot[record];
+            if (slot >= 0 && slot < record_count) {
+                if (piece == 0) {
+                    record_flags[slot] = any ? epoch | kFlagPartial : epoch;
+                    sum = make_float4(-sum.x, -sum.y, 0.5f * sum.z, sum.w);
+                }
+                else if (piece == 1) {
+                    sum.x *= 0.5f;
+                }
+                if (any) {
+                    store_partial(partials + static_cast<int64_t>(slot) * kPartialFloats + 4 * piece, sum);
                 }
             }
         }
-        __syncthreads();
-        if (valid && slot >= 0 && slot < record_count) {
-            const float4* source = reinterpret_cast<const float4*>(s_partial + lane * kPartialFloats);
-            float* destination = partials + slot * kPartialFloats;
-            store_partial(destination, source[0]);
-            store_partial(destination + 4, source[1]);
-            store_partial(destination + 8, source[2]);
-            record_flags[slot] = epoch;
+        if (kWaves == 1) {
+            __syncthreads();  // the next batch rewrites the sums (one wave: no barrier, an ordering)
         }
-        __syncthreads();
     }
-    // Records behind every pixel's last contributor contribute nothing; they get neither a
-    // partial nor this step's flag.
+    // Records after every pixel of the tile terminated (Stored: behind every pixel's last
+    // contributor) contribute nothing; they get neither a partial nor this step's flag.
 }
 
 __global__ __launch_bounds__(64) void wave_sum12_selftest_kernel(const float* input, float* output) {
@@ -631,11 +600,11 @@ int launch_splat_backward(gsn_context* context, const Camera& cam, int count, co
     if (!splats || !order || !groups_order || !record_flags) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
-    // The epoch runs 1..255. After a wrap, or in a newly allocated buffer, every byte is cleared
+    // The epoch runs 1..127 (the flag's eighth bit says that the record has a partial). After a wrap, or in a newly allocated buffer, every byte is cleared
     // first, so that a stale byte never equals the current epoch.
     uint8_t next = static_cast<uint8_t>(context->record_epoch + 1);
     const size_t flag_bytes = context->slot_bytes[kSlotRecordFlags];
-    if (next == 0 || context->record_flags_cleared != record_flags ||
+    if (next == kFlagPartial || context->record_flags_cleared != record_flags ||
         context->record_flags_cleared_bytes != flag_bytes) {
         int64_t words = static_cast<int64_t>(flag_bytes / 4);
         clear_flags_kernel<<<grid_for(words, 256), 256, 0, context->stream>>>(reinterpret_cast<uint32_t*>(record_flags),
@@ -657,15 +626,22 @@ int launch_splat_backward(gsn_context* context, const Camera& cam, int count, co
             record_offsets, buffers));
     }
     *gaussian_order = groups_order;
-    if (stored) {
-        raster_backward_stored_kernel<<<static_cast<unsigned>(tiles), 64, 0, context->stream>>>(ids, tile_offsets,
-            splats, order, cam, stored->final_transmittance, stored->last_contributor, image_gradients,
-            stored->background[0], stored->background[1], stored->background[2], partials, record_flags, next,
-            record_count);
-        return check_launch("raster_backward_stored_kernel");
+    auto launch = [&](auto kernel, int waves) {
+        kernel<<<static_cast<unsigned>(tiles), 64 * waves, 0, context->stream>>>(ids, tile_offsets, splats, order, cam,
+            image, stored ? stored->final_transmittance : nullptr, stored ? stored->last_contributor : nullptr,
+            image_gradients, stored ? stored->background[0] : 0.0f, stored ? stored->background[1] : 0.0f,
+            stored ? stored->background[2] : 0.0f, partials, record_flags, next, record_count);
+    };
+    // Four waves per tile while the tiles are few, one otherwise. Measured (us, four / two / one wave
+    // per tile): 256 tiles 102 / 156 / 226, 1,024 tiles 110 / 161 / 236, 4,056 tiles 274 / 240 / 238,
+    // 8,160 tiles 468 / 389 / 345; with one wave per tile and ten lane reads per splat the same images
+    // took 241, 241, 256 and 397. Stored form, 4,108 tiles: 259 / 233 / 204, before 236.
+    if (tiles <= 3072) {
+        stored ? launch(raster_backward_kernel<1, true>, 4) : launch(raster_backward_kernel<1, false>, 4);
     }
-    raster_backward_kernel<<<static_cast<unsigned>(tiles), 64, 0, context->stream>>>(ids, tile_offsets, splats, order,
-        cam, image, image_gradients, partials, record_flags, next, record_count);
+    else {
+        stored ? launch(raster_backward_kernel<4, true>, 1) : launch(raster_backward_kernel<4, false>, 1);
+    }
     return check_launch("raster_backward_kernel");
 }
 
