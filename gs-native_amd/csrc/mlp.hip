@@ -2,12 +2,15 @@
 // keep / clone / split) with BF16 weights and FP32 accumulation on gfx950 MFMA
 // (v_mfma_f32_32x32x16_bf16). No counterpart in the reference.
 //
-// One 64-lane workgroup processes tiles of 32 samples. Every GEMM of a tile is a few 32x32x16
-// MFMAs with both operands staged in LDS "K-contiguous" (A[m][k], B[n][k]), so each lane loads
-// its 8-element operand fragment with one 16-byte LDS read:
-//   A fragment: row (l & 31) of the M block, K elements 8 * (l >> 5) .. + 7 of the K chunk,
-//   B fragment: row (l & 31) of the N block, same K elements,
-//   D (f32x16): lane l holds column (l & 31), register v holds row 8 (v >> 2) + 4 (l >> 5) + (v & 3).
+// A wave processes tiles of 32 samples with everything in registers. An operand of a 32x32x16
+// product, A (rows) or B (columns), has the same form: lane l holds row (column) l & 31 and its K
+// elements 8 * (l >> 5) .. + 7 of the 16-element chunk; the result has column l & 31 in lane l and
+// row 8 (v >> 2) + 4 (l >> 5) + (v & 3) in register v. So mfma(weights, samples) gives samples in
+// lanes and features in registers ("by sample"), mfma(samples, weights) the other way round ("by
+// feature"), with the same bits; and a result whose lane is the next product's row becomes its
+// operand by converting to BF16 and exchanging four-element pieces between the wave's halves
+// (operand_chunk). No transposition through LDS, and weights stay in registers across tiles. (Staging
+// both layouts of weights and activations in LDS took 58 KB per one-wave workgroup, two waves per CU.)
 // Forward: Z1 = X W1^T + b1, A1 = relu(Z1); Z2 = A1 W2^T + b2, A2 = relu(Z2); Z3 = A2 W3^T + b3.
 // Backward (softmax cross-entropy): dZ3 = w (softmax(Z3) - onehot) / sum(w); dW3 = dZ3^T A2;
 // dA2 = dZ3 W3; dZ2 = dA2 [Z2 > 0]; dW2 = dZ2^T A1; dA1 = dZ2 W2; dZ1 = dA1 [Z1 > 0];
@@ -16,6 +19,7 @@
 // reduced in a fixed order by the Adam kernel (deterministic).
 #include "gsn_internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace gsn {
@@ -49,317 +53,451 @@ __device__ __forceinline__ int d_row(int lane, int v) {
     return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3);
 }
 
-__device__ __forceinline__ bf16x8 fragment(const __bf16* base, int row, int row_stride, int k0) {
-    return *reinterpret_cast<const bf16x8*>(base + row * row_stride + k0);
+// Chunk c (0, 1) of the operand that continues a 32x32 result: K elements 16 c .. 16 c + 15 of the
+// result's rows. Per half the lane holds rows 16 c + 4 h + (0..3) and 16 c + 8 + 4 h + (0..3); the
+// swap gives half 0 the first eight and half 1 the last eight.
+__device__ __forceinline__ bf16x8 operand_chunk(const float (&values)[16], int c) {
+    union Pieces {
+        __bf16 b[8];
+        uint32_t u[4];
+        bf16x8 v;
+    } piece;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        piece.b[i] = static_cast<__bf16>(values[8 * c + i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        auto swapped = __builtin_amdgcn_permlane32_swap(piece.u[i], piece.u[2 + i], false, false);
+        piece.u[i] = swapped[0];
+        piece.u[2 + i] = swapped[1];
+    }
+    return piece.v;
 }
 
-struct alignas(16) Weights {
-    __bf16 w1[kHidden * kIn];        // [o][k]
-    __bf16 w2[kHidden * kHidden];    // [o][i]
-    __bf16 w2t[kHidden * kHidden];   // [i][o]
-    __bf16 w3[32 * kHidden];         // [c][i], rows 3..31 zero
-    __bf16 w3t[kHidden * 16];        // [i][c], c 3..15 zero
+__device__ __forceinline__ bf16x8 zero_operand() {
+    bf16x8 zero = {};
+    return zero;
+}
+
+// Sixteen bytes from an address with no alignment beyond its elements' (the caller's buffers): one
+// wide load, which global memory serves at any element address.
+template<typename Wide, typename Element>
+__device__ __forceinline__ Wide load_wide(const Element* address) {
+    Wide value;
+    __builtin_memcpy(&value, address, sizeof(value));
+    return value;
+}
+
+// Operands of the weight matrices, one row of the matrix per lane.
+struct ForwardWeights {
+    bf16x8 w1[2];     // rows 32 b + l, K = the 16 inputs
+    bf16x8 w2[2][4];  // rows 32 b + l, K chunks of the 64 hidden units
+    bf16x8 w3[4];     // rows l (3..31 zero padding), K chunks
 };
 
-struct alignas(16) Activations {
-    __bf16 x[32 * kIn];         // [m][k]
-    __bf16 xt[32 * 32];         // [k][m], k 16..31 zero
-    __bf16 a1[32 * kHidden];    // [m][i]
-    __bf16 a1t[kHidden * 32];   // [i][m]
-    __bf16 a2[32 * kHidden];
-    __bf16 a2t[kHidden * 32];
-    __bf16 dz3[32 * 16];        // [m][c]
-    __bf16 dz3t[32 * 32];       // [c][m], c 3..31 zero
-    __bf16 dz2[32 * kHidden];   // [m][o]
-    __bf16 dz2t[kHidden * 32];  // [o][m]
-    __bf16 dz1t[kHidden * 32];  // [o][m]
-    float logits[32 * 4];
+__device__ __forceinline__ ForwardWeights load_forward_weights(const __bf16* __restrict__ weights) {
+    const int lane = threadIdx.x & 63;
+    const int row = lane & 31, k8 = (lane >> 5) * 8;
+    ForwardWeights w;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        w.w1[b] = load_wide<bf16x8>(weights + kBfW1 + (32 * b + row) * kIn + k8);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            w.w2[b][c] = load_wide<bf16x8>(weights + kBfW2 + (32 * b + row) * kHidden + 16 * c + k8);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        w.w3[c] = load_wide<bf16x8>(weights + kBfW3 + row * kHidden + 16 * c + k8);
+    }
+    return w;
+}
+
+// A tile's inputs by sample: lane's sample, inputs 8 h .. + 7 (zero past the last sample).
+struct TileInputs {
+    float4 low, high;
 };
 
-__device__ void load_weights(Weights& s, const __bf16* __restrict__ weights) {
-    const int t = threadIdx.x;
-    for (int i = t; i < kHidden * kIn; i += 64) {
-        s.w1[i] = weights[kBfW1 + i];
+__device__ __forceinline__ TileInputs load_inputs(const float* __restrict__ features, int64_t first, int count) {
+    const int lane = threadIdx.x & 63;
+    const int64_t sample = first + (lane & 31);
+    TileInputs x;
+    x.low = x.high = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (sample < count) {
+        const float* row = features + sample * kIn + (lane >> 5) * 8;
+        x.low = load_wide<float4>(row);
+        x.high = load_wide<float4>(row + 4);
     }
-    for (int i = t; i < kHidden * kHidden; i += 64) {
-        __bf16 w = weights[kBfW2 + i];
-        s.w2[i] = w;
-        int o = i / kHidden, j = i % kHidden;
-        s.w2t[j * kHidden + o] = w;
-    }
-    for (int i = t; i < 32 * kHidden; i += 64) {
-        __bf16 w = weights[kBfW3 + i];
-        s.w3[i] = w;
-    }
-    for (int i = t; i < kHidden * 16; i += 64) {
-        int j = i / 16, c = i % 16;
-        s.w3t[i] = c < kClasses ? weights[kBfW3 + c * kHidden + j] : static_cast<__bf16>(0.0f);
-    }
-    __syncthreads();
+    return x;
 }
 
-// Stages one tile of features (rows past `count` are zero) in both layouts.
-__device__ void load_tile(Activations& s, const float* __restrict__ features, int64_t first, int count) {
-    const int t = threadIdx.x;
-    for (int i = t; i < 32 * kIn; i += 64) {
-        int m = i / kIn, k = i % kIn;
-        float v = first + m < count ? features[(first + m) * kIn + k] : 0.0f;
-        __bf16 b = static_cast<__bf16>(v);
-        s.x[i] = b;
-        s.xt[k * 32 + m] = b;
+__device__ __forceinline__ bf16x8 input_operand(const TileInputs& x) {
+    const float v[8] = {x.low.x, x.low.y, x.low.z, x.low.w, x.high.x, x.high.y, x.high.z, x.high.w};
+    bf16x8 out;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        out[i] = static_cast<__bf16>(v[i]);
     }
-    for (int i = t; i < 16 * 32; i += 64) {
-        s.xt[16 * 32 + i] = static_cast<__bf16>(0.0f);
-    }
-    __syncthreads();
+    return out;
 }
 
-// Forward of one tile; leaves Z1/Z2 in registers (D layout) for the ReLU masks and the logits in
-// LDS.
-__device__ void forward_tile(Activations& s, const Weights& w, const float* __restrict__ biases, f32x16 z1[2],
-    f32x16 z2[2]) {
-    const int lane = threadIdx.x;
-    const int n = lane & 31;
-    const int k8 = (lane >> 5) * 8;
-    for (int nb = 0; nb < 2; ++nb) {
-        f32x16 acc = {};
-        acc = mfma(fragment(s.x, n, kIn, k8), fragment(w.w1, nb * 32 + n, kIn, k8), acc);
-        float bias = biases[kB1 + nb * 32 + n];
-        for (int v = 0; v < 16; ++v) {
-            acc[v] += bias;
-            int m = d_row(lane, v);
-            __bf16 a = static_cast<__bf16>(fmaxf(acc[v], 0.0f));
-            s.a1[m * kHidden + nb * 32 + n] = a;
-            s.a1t[(nb * 32 + n) * 32 + m] = a;
-        }
-        z1[nb] = acc;
+// values += bias of each row of a by-sample result (rows 32 b + d_row); bias is in LDS, four
+// consecutive rows a read.
+__device__ __forceinline__ void add_row_bias(float (&values)[16], const f32x16& acc, const float* bias, int b) {
+    const int half = (threadIdx.x >> 5) & 1;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const float4 four = *reinterpret_cast<const float4*>(bias + 32 * b + 8 * g + 4 * half);
+        values[4 * g] = acc[4 * g] + four.x;
+        values[4 * g + 1] = acc[4 * g + 1] + four.y;
+        values[4 * g + 2] = acc[4 * g + 2] + four.z;
+        values[4 * g + 3] = acc[4 * g + 3] + four.w;
     }
-    __syncthreads();
-    for (int nb = 0; nb < 2; ++nb) {
-        f32x16 acc = {};
-        for (int kc = 0; kc < 4; ++kc) {
-            acc = mfma(fragment(s.a1, n, kHidden, kc * 16 + k8), fragment(w.w2, nb * 32 + n, kHidden, kc * 16 + k8), acc);
-        }
-        float bias = biases[kB2 + nb * 32 + n];
-        for (int v = 0; v < 16; ++v) {
-            acc[v] += bias;
-            int m = d_row(lane, v);
-            __bf16 a = static_cast<__bf16>(fmaxf(acc[v], 0.0f));
-            s.a2[m * kHidden + nb * 32 + n] = a;
-            s.a2t[(nb * 32 + n) * 32 + m] = a;
-        }
-        z2[nb] = acc;
+}
+
+__device__ __forceinline__ void relu(const float (&in)[16], float (&out)[16]) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        out[v] = fmaxf(in[v], 0.0f);
     }
-    __syncthreads();
+}
+
+// The by-sample hidden layers of a tile: pre-activations z (before the ReLU) of both layers and the
+// operands of the activations.
+struct HiddenLayers {
+    bf16x8 a1[4], a2[4];
+};
+
+__device__ __forceinline__ void hidden_layers(const ForwardWeights& w, const float* bias1, const float* bias2, bf16x8 x,
+    HiddenLayers& layers, float (&z2)[2][16]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        float z[16], a[16];
+        add_row_bias(z, mfma(w.w1[b], x, f32x16{}), bias1, b);
+        relu(z, a);
+        layers.a1[2 * b] = operand_chunk(a, 0);
+        layers.a1[2 * b + 1] = operand_chunk(a, 1);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        f32x16 acc = {};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            acc = mfma(w.w2[b][c], layers.a1[c], acc);
+        }
+        float a[16];
+        add_row_bias(z2[b], acc, bias2, b);
+        relu(z2[b], a);
+        layers.a2[2 * b] = operand_chunk(a, 0);
+        layers.a2[2 * b + 1] = operand_chunk(a, 1);
+    }
+}
+
+// The logits of lane's sample: classes 0..2 in registers 0..2 of the lanes below 32.
+__device__ __forceinline__ f32x16 output_layer(const ForwardWeights& w, const HiddenLayers& layers) {
     f32x16 acc = {};
-    for (int kc = 0; kc < 4; ++kc) {
-        acc = mfma(fragment(s.a2, n, kHidden, kc * 16 + k8), fragment(w.w3, n, kHidden, kc * 16 + k8), acc);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        acc = mfma(w.w3[c], layers.a2[c], acc);
     }
-    if (n < kClasses) {
-        float bias = biases[kB3 + n];
-        for (int v = 0; v < 16; ++v) {
-            s.logits[d_row(lane, v) * 4 + n] = acc[v] + bias;
-        }
+    return acc;
+}
+
+// The two hidden layers' biases in LDS; every wave of the workgroup reads them.
+__device__ __forceinline__ void stage_biases(const float* __restrict__ biases, float* bias1, float* bias2) {
+    if (threadIdx.x < kHidden) {
+        bias1[threadIdx.x] = biases[kB1 + threadIdx.x];
+        bias2[threadIdx.x] = biases[kB2 + threadIdx.x];
     }
     __syncthreads();
 }
 
-__global__ __launch_bounds__(64) void mlp_forward_kernel(const float* __restrict__ features, int count,
+constexpr int kMlpWaves = 4;  // per workgroup
+
+// 76 bytes and 10.6 kFLOP a sample: bound by memory once enough waves are in flight; the next tile's
+// inputs are loaded while one is computed. 500K samples: 205 us with tiles
+// staged through LDS by one wave per workgroup, 21 us so.
+__global__ __launch_bounds__(64 * kMlpWaves) void mlp_forward_kernel(const float* __restrict__ features, int count,
     const __bf16* __restrict__ weights, const float* __restrict__ biases, float* __restrict__ logits) {
-    __shared__ Weights w;
-    __shared__ Activations s;
-    load_weights(w, weights);
+    __shared__ __align__(16) float bias1[kHidden], bias2[kHidden];
+    stage_biases(biases, bias1, bias2);
+    const ForwardWeights w = load_forward_weights(weights);
+    const float bias3[kClasses] = {biases[kB3], biases[kB3 + 1], biases[kB3 + 2]};
+    const int lane = threadIdx.x & 63;
     const int tiles = (count + 31) / 32;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        int64_t first = static_cast<int64_t>(tile) * 32;
-        load_tile(s, features, first, count);
-        f32x16 z1[2], z2[2];
-        forward_tile(s, w, biases, z1, z2);
-        for (int i = threadIdx.x; i < 32 * kClasses; i += 64) {
-            int m = i / kClasses, c = i % kClasses;
-            if (first + m < count) {
-                logits[(first + m) * kClasses + c] = s.logits[m * 4 + c];
+    const int stride = static_cast<int>(gridDim.x) * kMlpWaves;
+    int tile = static_cast<int>(blockIdx.x) * kMlpWaves + static_cast<int>(threadIdx.x >> 6);
+    TileInputs next = load_inputs(features, static_cast<int64_t>(tile) * 32, count);
+    for (; tile < tiles; tile += stride) {
+        const bf16x8 x = input_operand(next);
+        next = load_inputs(features, (static_cast<int64_t>(tile) + stride) * 32, count);
+        HiddenLayers layers;
+        float z2[2][16];
+        hidden_layers(w, bias1, bias2, x, layers, z2);
+        const f32x16 out = output_layer(w, layers);
+        const int64_t sample = static_cast<int64_t>(tile) * 32 + lane;
+        if (lane < 32 && sample < count) {
+#pragma unroll
+            for (int c = 0; c < kClasses; ++c) {
+                logits[sample * kClasses + c] = out[c] + bias3[c];
             }
         }
-        __syncthreads();
     }
 }
 
-// Forward + backward over the workgroup's tiles; writes this workgroup's gradient sums
-// (parameter layout) and loss sum to partials[blockIdx.x].
-__global__ __launch_bounds__(64) void mlp_gradient_kernel(const float* __restrict__ features,
+// Forward + backward over the workgroup's tiles; writes its gradient sums (parameter layout) and
+// loss sum to partials[blockIdx.x]. A wave keeps its sums in registers (seven 32x32 results); at the
+// end the workgroup adds its waves' sums through LDS, wave by wave, so that every order is fixed.
+// Weight gradients sum over the samples, so their operands need samples as K: the by-feature
+// results, computed by a second product of the same operands in the other order. Bound by the chain of
+// products of a tile at four waves per CU; 65,536 samples: 75 us with the activations kept in LDS for
+// the transposed reads, 29 us so.
+__global__ __launch_bounds__(64 * kMlpWaves, 1) void mlp_gradient_kernel(const float* __restrict__ features,
     const int* __restrict__ labels, const float* __restrict__ sample_weights, int count, float weight_scale,
     const __bf16* __restrict__ weights, const float* __restrict__ biases, float* __restrict__ partials,
     float* __restrict__ loss_partials) {
-    __shared__ Weights w;
-    __shared__ Activations s;
-    load_weights(w, weights);
-    const int lane = threadIdx.x;
+    __shared__ __align__(16) float bias1[kHidden], bias2[kHidden];
+    __shared__ __align__(16) __bf16 s_dz3[kMlpWaves][kClasses][32];  // [class][sample]
+    __shared__ float s_sum[kParams + 1];                             // gradients, then the loss
+    stage_biases(biases, bias1, bias2);
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
     const int n = lane & 31;
-    const int k8 = (lane >> 5) * 8;
+    const int half = lane >> 5;
+    const int k8 = half * 8;
+    const ForwardWeights w = load_forward_weights(weights);
+    // Operands of the transposed matrices: rows are the hidden units 32 b + n.
+    bf16x8 w3t[2], w2t[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        w3t[b] = zero_operand();
+        if (half == 0) {
+#pragma unroll
+            for (int c = 0; c < kClasses; ++c) {
+                w3t[b][c] = weights[kBfW3 + c * kHidden + 32 * b + n];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                w2t[b][c][i] = weights[kBfW2 + (16 * c + k8 + i) * kHidden + 32 * b + n];
+            }
+        }
+    }
+    const float bias3[kClasses] = {biases[kB3], biases[kB3 + 1], biases[kB3 + 2]};
+    const float own_bias1[2] = {bias1[n], bias1[32 + n]}, own_bias2[2] = {bias2[n], bias2[32 + n]};
     f32x16 gw1[2] = {}, gw2[4] = {}, gw3[2] = {};
-    float gb1[2] = {0.0f, 0.0f}, gb2[2] = {0.0f, 0.0f}, gb3 = 0.0f;
+    float gb1[2] = {0.0f, 0.0f}, gb2[2] = {0.0f, 0.0f}, gb3[kClasses] = {0.0f, 0.0f, 0.0f};
     float loss = 0.0f;
     const int tiles = (count + 31) / 32;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        int64_t first = static_cast<int64_t>(tile) * 32;
-        load_tile(s, features, first, count);
-        f32x16 z1[2], z2[2];
-        forward_tile(s, w, biases, z1, z2);
+    for (int tile = blockIdx.x * kMlpWaves + wave; tile < tiles; tile += gridDim.x * kMlpWaves) {
+        const int64_t first = static_cast<int64_t>(tile) * 32;
+        const bf16x8 x = input_operand(load_inputs(features, first, count));
+        // The inputs by feature (lane = input, 16..31 zero): samples 16 c + 8 h .. + 7.
+        bf16x8 xt[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int64_t sample = first + 16 * c + k8 + i;
+                xt[c][i] = static_cast<__bf16>(n < kIn && sample < count ? features[sample * kIn + n] : 0.0f);
+            }
+        }
+        HiddenLayers layers;
+        float z2[2][16];
+        hidden_layers(w, bias1, bias2, x, layers, z2);
+        const f32x16 out = output_layer(w, layers);
         // Softmax cross-entropy, one lane per sample.
-        if (lane < 32) {
-            int m = lane;
-            bool valid = first + m < count;
-            float weight = valid ? (sample_weights ? sample_weights[first + m] : 1.0f) * weight_scale : 0.0f;
-            int label = valid ? labels[first + m] : 0;
-            float l0 = s.logits[m * 4], l1 = s.logits[m * 4 + 1], l2 = s.logits[m * 4 + 2];
-            float top = fmaxf(l0, fmaxf(l1, l2));
-            float e0 = __expf(l0 - top), e1 = __expf(l1 - top), e2 = __expf(l2 - top);
-            float sum = e0 + e1 + e2;
-            float p[3] = {e0 / sum, e1 / sum, e2 / sum};
-            float chosen = label == 0 ? l0 : (label == 1 ? l1 : l2);
+        bf16x8 dz3 = zero_operand();
+        if (half == 0) {
+            const bool valid = first + n < count;
+            const float weight = valid ? (sample_weights ? sample_weights[first + n] : 1.0f) * weight_scale : 0.0f;
+            const int label = valid ? labels[first + n] : 0;
+            const float l0 = out[0] + bias3[0], l1 = out[1] + bias3[1], l2 = out[2] + bias3[2];
+            const float top = fmaxf(l0, fmaxf(l1, l2));
+            const float e0 = __expf(l0 - top), e1 = __expf(l1 - top), e2 = __expf(l2 - top);
+            const float sum = e0 + e1 + e2;
+            const float p[3] = {e0 / sum, e1 / sum, e2 / sum};
+            const float chosen = label == 0 ? l0 : (label == 1 ? l1 : l2);
             if (valid) {
                 loss += weight * (top + __logf(sum) - chosen);
             }
-            for (int c = 0; c < 16; ++c) {
-                float g = c < kClasses ? weight * (p[c] - (c == label ? 1.0f : 0.0f)) : 0.0f;
-                __bf16 b = static_cast<__bf16>(g);
-                s.dz3[m * 16 + c] = b;
-            }
-            for (int c = 0; c < 32; ++c) {
-                s.dz3t[c * 32 + m] = c < kClasses ? s.dz3[m * 16 + c] : static_cast<__bf16>(0.0f);
+#pragma unroll
+            for (int c = 0; c < kClasses; ++c) {
+                dz3[c] = static_cast<__bf16>(weight * (p[c] - (c == label ? 1.0f : 0.0f)));
+                s_dz3[wave][c][n] = dz3[c];
+                gb3[c] += static_cast<float>(dz3[c]);
             }
         }
-        __syncthreads();
-        // db3, dW3 (M = class, N = hidden, K = samples).
-        if (lane < kClasses) {
-            for (int m = 0; m < 32; ++m) {
-                gb3 += static_cast<float>(s.dz3[m * 16 + lane]);
-            }
+        __builtin_amdgcn_wave_barrier();
+        bf16x8 dz3t[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            dz3t[c] = n < kClasses ? *reinterpret_cast<const bf16x8*>(&s_dz3[wave][n][16 * c + k8]) : zero_operand();
         }
-        for (int nb = 0; nb < 2; ++nb) {
-            for (int kc = 0; kc < 2; ++kc) {
-                gw3[nb] = mfma(fragment(s.dz3t, n, 32, kc * 16 + k8), fragment(s.a2t, nb * 32 + n, 32, kc * 16 + k8),
-                    gw3[nb]);
+        __builtin_amdgcn_wave_barrier();
+        // By feature: the activations of both layers, and dZ2 and dZ1 with them.
+        bf16x8 dz2[4], dz2t[2][2], a1t[2][2];
+        float z1t[2][16];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const f32x16 first_layer = mfma(x, w.w1[b], f32x16{});
+            f32x16 second_layer = {};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                second_layer = mfma(layers.a1[c], w.w2[b][c], second_layer);
             }
-        }
-        // dA2 = dZ3 W3 (M = samples, N = hidden, K = class padded to 16), masked by Z2 > 0.
-        for (int nb = 0; nb < 2; ++nb) {
-            f32x16 acc = {};
-            acc = mfma(fragment(s.dz3, n, 16, k8), fragment(w.w3t, nb * 32 + n, 16, k8), acc);
-            float column = 0.0f;
+            float z2t[16], a[16];
+#pragma unroll
             for (int v = 0; v < 16; ++v) {
-                float g = z2[nb][v] > 0.0f ? acc[v] : 0.0f;
-                __bf16 b = static_cast<__bf16>(g);
-                int m = d_row(lane, v);
-                s.dz2[m * kHidden + nb * 32 + n] = b;
-                s.dz2t[(nb * 32 + n) * 32 + m] = b;
-                column += static_cast<float>(b);
+                z1t[b][v] = first_layer[v] + own_bias1[b];
+                z2t[v] = second_layer[v] + own_bias2[b];
             }
-            gb2[nb] += column;
+            relu(z1t[b], a);
+            a1t[b][0] = operand_chunk(a, 0);
+            a1t[b][1] = operand_chunk(a, 1);
+            relu(z2t, a);
+            // dW3 (rows = class, columns = hidden, K = samples).
+            gw3[b] = mfma(dz3t[0], operand_chunk(a, 0), gw3[b]);
+            gw3[b] = mfma(dz3t[1], operand_chunk(a, 1), gw3[b]);
+            // dA2 = dZ3 W3, masked by Z2 > 0: by sample for dA1, by feature for dW2.
+            const f32x16 da2 = mfma(w3t[b], dz3, f32x16{});
+            const f32x16 da2t = mfma(dz3, w3t[b], f32x16{});
+            float g[16], gt[16], column = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                g[v] = z2[b][v] > 0.0f ? da2[v] : 0.0f;
+                gt[v] = z2t[v] > 0.0f ? da2t[v] : 0.0f;
+                column += static_cast<float>(static_cast<__bf16>(gt[v]));
+            }
+            gb2[b] += column;
+            dz2[2 * b] = operand_chunk(g, 0);
+            dz2[2 * b + 1] = operand_chunk(g, 1);
+            dz2t[b][0] = operand_chunk(gt, 0);
+            dz2t[b][1] = operand_chunk(gt, 1);
         }
-        __syncthreads();
-        // dW2 (M = out, N = in, K = samples).
+        // dW2 (rows = out, columns = in, K = samples).
+#pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-                for (int kc = 0; kc < 2; ++kc) {
-                    gw2[mb * 2 + nb] = mfma(fragment(s.dz2t, mb * 32 + n, 32, kc * 16 + k8),
-                        fragment(s.a1t, nb * 32 + n, 32, kc * 16 + k8), gw2[mb * 2 + nb]);
+                gw2[mb * 2 + nb] = mfma(dz2t[mb][0], a1t[nb][0], gw2[mb * 2 + nb]);
+                gw2[mb * 2 + nb] = mfma(dz2t[mb][1], a1t[nb][1], gw2[mb * 2 + nb]);
+            }
+        }
+        // dA1 = dZ2 W2 by feature, masked by Z1 > 0; dW1 (rows = out, columns = input, K = samples).
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            f32x16 acc = {};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                acc = mfma(dz2[c], w2t[b][c], acc);
+            }
+            float g[16], column = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                g[v] = z1t[b][v] > 0.0f ? acc[v] : 0.0f;
+                column += static_cast<float>(static_cast<__bf16>(g[v]));
+            }
+            gb1[b] += column;
+            gw1[b] = mfma(operand_chunk(g, 0), xt[0], gw1[b]);
+            gw1[b] = mfma(operand_chunk(g, 1), xt[1], gw1[b]);
+        }
+    }
+    // Sums over the workgroup's waves, in wave order. A result's lane column is n, its register rows
+    // d_row(lane, v); a bias's two halves of rows meet first.
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        gb1[b] += __shfl_xor(gb1[b], 32);
+        gb2[b] += __shfl_xor(gb2[b], 32);
+    }
+#pragma unroll
+    for (int offset = 16; offset > 0; offset >>= 1) {
+        loss += __shfl_xor(loss, offset);
+#pragma unroll
+        for (int c = 0; c < kClasses; ++c) {
+            gb3[c] += __shfl_xor(gb3[c], offset);
+        }
+    }
+    for (int turn = 0; turn < kMlpWaves; ++turn) {
+        if (wave == turn) {
+            auto add = [&](int at, float value) { s_sum[at] = turn == 0 ? value : s_sum[at] + value; };
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int row = d_row(lane, v);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    if (n < kIn) {
+                        add(kW1 + (32 * b + row) * kIn + n, gw1[b][v]);
+                    }
+                    add(kW2 + (32 * b + row) * kHidden + n, gw2[2 * b][v]);
+                    add(kW2 + (32 * b + row) * kHidden + 32 + n, gw2[2 * b + 1][v]);
+                    if (row < kClasses) {
+                        add(kW3 + row * kHidden + 32 * b + n, gw3[b][v]);
+                    }
+                }
+            }
+            if (half == 0) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    add(kB1 + 32 * b + n, gb1[b]);
+                    add(kB2 + 32 * b + n, gb2[b]);
+                }
+                if (n < kClasses) {
+                    add(kB3 + n, n == 0 ? gb3[0] : (n == 1 ? gb3[1] : gb3[2]));
+                }
+                if (n == 0) {
+                    add(kParams, loss);
                 }
             }
         }
-        // dA1 = dZ2 W2 (M = samples, N = in, K = out), masked by Z1 > 0.
-        for (int nb = 0; nb < 2; ++nb) {
-            f32x16 acc = {};
-            for (int kc = 0; kc < 4; ++kc) {
-                acc = mfma(fragment(s.dz2, n, kHidden, kc * 16 + k8), fragment(w.w2t, nb * 32 + n, kHidden, kc * 16 + k8),
-                    acc);
-            }
-            float column = 0.0f;
-            for (int v = 0; v < 16; ++v) {
-                float g = z1[nb][v] > 0.0f ? acc[v] : 0.0f;
-                __bf16 b = static_cast<__bf16>(g);
-                s.dz1t[(nb * 32 + n) * 32 + d_row(lane, v)] = b;
-                column += static_cast<float>(b);
-            }
-            gb1[nb] += column;
-        }
-        __syncthreads();
-        // dW1 (M = out, N = input padded to 32, K = samples).
-        for (int mb = 0; mb < 2; ++mb) {
-            for (int kc = 0; kc < 2; ++kc) {
-                gw1[mb] = mfma(fragment(s.dz1t, mb * 32 + n, 32, kc * 16 + k8), fragment(s.xt, n, 32, kc * 16 + k8),
-                    gw1[mb]);
-            }
-        }
         __syncthreads();
     }
-    // Write this workgroup's sums. D layout: lane column n, register rows d_row(lane, v).
     float* out = partials + static_cast<int64_t>(blockIdx.x) * kParams;
-    for (int mb = 0; mb < 2; ++mb) {
-        for (int v = 0; v < 16; ++v) {
-            int o = mb * 32 + d_row(lane, v);
-            if (n < kIn) {
-                out[kW1 + o * kIn + n] = gw1[mb][v];
-            }
-        }
+    for (int i = threadIdx.x; i < kParams; i += 64 * kMlpWaves) {
+        out[i] = s_sum[i];
     }
-    for (int mb = 0; mb < 2; ++mb) {
-        for (int nb = 0; nb < 2; ++nb) {
-            for (int v = 0; v < 16; ++v) {
-                int o = mb * 32 + d_row(lane, v);
-                out[kW2 + o * kHidden + nb * 32 + n] = gw2[mb * 2 + nb][v];
-            }
-        }
-    }
-    for (int nb = 0; nb < 2; ++nb) {
-        for (int v = 0; v < 16; ++v) {
-            int c = d_row(lane, v);
-            if (c < kClasses) {
-                out[kW3 + c * kHidden + nb * 32 + n] = gw3[nb][v];
-            }
-        }
-    }
-    // Bias sums: lanes n and n + 32 hold the two row groups of the same column.
-    __shared__ float bias_sums[2][2][64];
-    for (int nb = 0; nb < 2; ++nb) {
-        bias_sums[0][nb][lane] = gb1[nb];
-        bias_sums[1][nb][lane] = gb2[nb];
-    }
-    __syncthreads();
-    if (lane < 32) {
-        for (int nb = 0; nb < 2; ++nb) {
-            out[kB1 + nb * 32 + lane] = bias_sums[0][nb][lane] + bias_sums[0][nb][lane + 32];
-            out[kB2 + nb * 32 + lane] = bias_sums[1][nb][lane] + bias_sums[1][nb][lane + 32];
-        }
-    }
-    if (lane < kClasses) {
-        out[kB3 + lane] = gb3;
-    }
-    __shared__ float losses[64];
-    losses[lane] = loss;
-    __syncthreads();
-    if (lane == 0) {
-        float total = 0.0f;
-        for (int i = 0; i < 32; ++i) {
-            total += losses[i];
-        }
-        loss_partials[blockIdx.x] = total;
+    if (threadIdx.x == 0) {
+        loss_partials[blockIdx.x] = s_sum[kParams];
     }
 }
 
-// Sums the per-workgroup gradients in a fixed order, applies Adam to the FP32 master parameters
+// Sums the workgroups' gradients in a fixed order, applies Adam to the FP32 master parameters
 // and refreshes the BF16 weight copy. gradients_out (optional) receives the summed gradients.
-__global__ __launch_bounds__(256) void mlp_adam_kernel(const float* __restrict__ partials, int groups,
-    float* __restrict__ params, float* __restrict__ first, float* __restrict__ second, __bf16* __restrict__ weights,
-    float learning_rate, float first_correction, float second_correction, float* __restrict__ gradients_out) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kParams) {
+// A workgroup has kAdamParams parameters and kAdamSegments runs of the partials' rows; each run is
+// added by its own threads (coalesced, many loads in flight), then the runs in order. (One thread
+// per parameter over 1,024 rows one after another took 245 us; so, over 256 rows, 4.8.)
+constexpr int kAdamParams = 32;
+constexpr int kAdamSegments = 16;
+
+__global__ __launch_bounds__(kAdamParams * kAdamSegments) void mlp_adam_kernel(const float* __restrict__ partials,
+    int groups, float* __restrict__ params, float* __restrict__ first, float* __restrict__ second,
+    __bf16* __restrict__ weights, float learning_rate, float first_correction, float second_correction,
+    float* __restrict__ gradients_out) {
+    __shared__ float s_sum[kAdamSegments][kAdamParams];
+    const int segment = threadIdx.x / kAdamParams;
+    const int p = blockIdx.x * kAdamParams + threadIdx.x % kAdamParams;
+    const int rows = (groups + kAdamSegments - 1) / kAdamSegments;
+    const int begin = min(segment * rows, groups), end = min(begin + rows, groups);
+    float sum = 0.0f;
+    if (p < kParams) {
+#pragma unroll 8
+        for (int row = begin; row < end; ++row) {
+            sum += partials[static_cast<int64_t>(row) * kParams + p];
+        }
+    }
+    s_sum[segment][threadIdx.x % kAdamParams] = sum;
+    __syncthreads();
+    if (segment != 0 || p >= kParams) {
         return;
     }
     float g = 0.0f;
-    for (int b = 0; b < groups; ++b) {
-        g += partials[static_cast<int64_t>(b) * kParams + p];
+#pragma unroll
+    for (int k = 0; k < kAdamSegments; ++k) {
+        g += s_sum[k][threadIdx.x];
     }
     if (gradients_out) {
         gradients_out[p] = g;
@@ -390,10 +528,16 @@ __global__ void mlp_zero_padding_kernel(__bf16* weights) {
     }
 }
 
-int mlp_groups(int count) {
-    int tiles = (count + 31) / 32;
-    return tiles < 1024 ? (tiles > 0 ? tiles : 1) : 1024;
+// Workgroups of kMlpWaves tiles each, at most `most`; beyond that the waves take several tiles.
+int mlp_groups(int count, int most) {
+    const int64_t tiles = (static_cast<int64_t>(count) + 31) / 32;
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((tiles + kMlpWaves - 1) / kMlpWaves, most)));
 }
+
+// Forward: four workgroups a CU hide the loads. Training: one a CU, whose waves' gradient sums take
+// most of the registers; more would also mean more partials to add.
+constexpr int kForwardGroups = 1024;
+constexpr int kTrainingGroups = 256;
 
 } // namespace
 } // namespace gsn
@@ -415,7 +559,7 @@ extern "C" int gsn_mlp_sync_weights(gsn_context* context, const float* params, u
     mlp_zero_padding_kernel<<<grid_for((32 - kClasses) * kHidden, 256), 256, 0, context->stream>>>(
         reinterpret_cast<__bf16*>(weights));
     GSN_TRY(check_launch("mlp_zero_padding_kernel"));
-    mlp_adam_kernel<<<grid_for(kParams, 256), 256, 0, context->stream>>>(nullptr, 0, const_cast<float*>(params),
+    mlp_adam_kernel<<<grid_for(kParams, kAdamParams), kAdamParams * kAdamSegments, 0, context->stream>>>(nullptr, 0, const_cast<float*>(params),
         nullptr, nullptr, reinterpret_cast<__bf16*>(weights), 0.0f, 0.0f, 0.0f, nullptr);
     return check_launch("mlp_adam_kernel");
 }
@@ -429,7 +573,7 @@ extern "C" int gsn_mlp_forward(gsn_context* context, const float* features, int 
     if (count == 0) {
         return GSN_OK;
     }
-    mlp_forward_kernel<<<mlp_groups(count), 64, 0, context->stream>>>(features, count,
+    mlp_forward_kernel<<<mlp_groups(count, kForwardGroups), 64 * kMlpWaves, 0, context->stream>>>(features, count,
         reinterpret_cast<const __bf16*>(weights), params, logits);
     return check_launch("mlp_forward_kernel");
 }
@@ -442,19 +586,19 @@ extern "C" int gsn_mlp_train_step(gsn_context* context, const float* features, c
         !(learning_rate >= 0.0f) || (learning_rate > 0.0f && (!first || !second))) {
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_mlp_train_step: invalid arguments");
     }
-    int groups = mlp_groups(count);
+    int groups = mlp_groups(count, kTrainingGroups);
     float* partials = static_cast<float*>(scratch(context, kSlotMisc, static_cast<size_t>(groups) * (kParams + 1) * 4));
     if (!partials) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
     float* loss_partials = partials + static_cast<size_t>(groups) * kParams;
     float weight_scale = 1.0f / static_cast<float>(count);
-    mlp_gradient_kernel<<<groups, 64, 0, context->stream>>>(features, labels, sample_weights, count, weight_scale,
+    mlp_gradient_kernel<<<groups, 64 * kMlpWaves, 0, context->stream>>>(features, labels, sample_weights, count, weight_scale,
         reinterpret_cast<const __bf16*>(weights), params, partials, loss_partials);
     GSN_TRY(check_launch("mlp_gradient_kernel"));
     float c1 = static_cast<float>(1.0 / (1.0 - std::pow(0.9, step)));
     float c2 = static_cast<float>(1.0 / (1.0 - std::pow(0.999, step)));
-    mlp_adam_kernel<<<grid_for(kParams, 256), 256, 0, context->stream>>>(partials, groups, params, first, second,
+    mlp_adam_kernel<<<grid_for(kParams, kAdamParams), kAdamParams * kAdamSegments, 0, context->stream>>>(partials, groups, params, first, second,
         reinterpret_cast<__bf16*>(weights), learning_rate, c1, c2, gradients_out);
     GSN_TRY(check_launch("mlp_adam_kernel"));
     if (loss_out) {
