@@ -94,7 +94,7 @@ int gsn_context_create(gsn_context** context) {
         status = gsn::check_hip(hipStreamCreate(&created->stream), "hipStreamCreate");
     }
     if (status == GSN_OK) {
-        status = gsn::check_hip(hipHostMalloc(&created->pinned, 256, hipHostMallocDefault), "hipHostMalloc");
+        status = gsn::check_hip(hipHostMalloc(&created->pinned, kPinnedBytes, hipHostMallocDefault), "hipHostMalloc");
     }
     if (status == GSN_OK) {
         status = gsn::check_hip(hipEventCreateWithFlags(&created->readback_event, hipEventDisableTiming),

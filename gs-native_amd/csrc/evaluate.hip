@@ -5,27 +5,61 @@
 // Integer work: the sum is exact, so the result does not depend on the summation order.
 #include "gsn_internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace gsn {
 namespace {
 
-constexpr int kEvalThreads = 256;
+// At most one workgroup per CU: each leaves one sum and the host adds them (integers, exact in any
+// order). With 8,192 workgroups adding to one 64-bit address the atomics alone took 100 us.
+constexpr int kEvalThreads = 1024;
+constexpr unsigned kEvalGroups = 256;
 
+__device__ __forceinline__ int quantize(float value) {
+    const float v = fminf(fmaxf(value, 0.0f), 1.0f);
+    return static_cast<int>(rintf(v * 255.0f));
+}
+
+// Bound by memory (18 bytes a pixel): groups of four values as one 16-byte and two 4-byte accesses
+// where the caller's buffers are aligned for them (Wide), value by value otherwise and at the end.
+// 1332x876: 102 us with one atomic sum and a value a thread, 6.3 us so.
+template<bool Wide>
 __global__ __launch_bounds__(kEvalThreads) void quantized_error_kernel(const float* __restrict__ image,
     const uint8_t* __restrict__ target, uint8_t* __restrict__ quantized, int64_t values,
-    unsigned long long* __restrict__ sse) {
+    unsigned long long* __restrict__ sums) {
     __shared__ unsigned long long partial[kEvalThreads / 64];
+    const int64_t thread = static_cast<int64_t>(blockIdx.x) * kEvalThreads + threadIdx.x;
+    const int64_t threads = static_cast<int64_t>(gridDim.x) * kEvalThreads;
     unsigned long long sum = 0;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kEvalThreads + threadIdx.x; i < values;
-         i += static_cast<int64_t>(gridDim.x) * kEvalThreads) {
-        float v = fminf(fmaxf(image[i], 0.0f), 1.0f);
-        int q = static_cast<int>(rintf(v * 255.0f));
-        if (quantized) {
-            quantized[i] = static_cast<uint8_t>(q);
-        }
-        int d = q - static_cast<int>(target[i]);
+    auto one = [&](float value, int goal) {
+        const int q = quantize(value);
+        const int d = q - goal;
         sum += static_cast<unsigned long long>(d * d);
+        return static_cast<uint8_t>(q);
+    };
+    int64_t done = 0;
+    if (Wide) {
+        const int64_t fours = values / 4;
+        for (int64_t i = thread; i < fours; i += threads) {
+            const float4 v = reinterpret_cast<const float4*>(image)[i];
+            const uchar4 t = reinterpret_cast<const uchar4*>(target)[i];
+            uchar4 q;
+            q.x = one(v.x, t.x);
+            q.y = one(v.y, t.y);
+            q.z = one(v.z, t.z);
+            q.w = one(v.w, t.w);
+            if (quantized) {
+                reinterpret_cast<uchar4*>(quantized)[i] = q;
+            }
+        }
+        done = fours * 4;
+    }
+    for (int64_t i = done + thread; i < values; i += threads) {
+        const uint8_t q = one(image[i], static_cast<int>(target[i]));
+        if (quantized) {
+            quantized[i] = q;
+        }
     }
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {
@@ -40,7 +74,7 @@ __global__ __launch_bounds__(kEvalThreads) void quantized_error_kernel(const flo
         for (int w = 0; w < kEvalThreads / 64; ++w) {
             block += partial[w];
         }
-        atomicAdd(sse, block);
+        sums[blockIdx.x] = block;
     }
 }
 
@@ -54,18 +88,26 @@ extern "C" int gsn_image_quantized_error(gsn_context* context, int width, int he
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_image_quantized_error: invalid arguments");
     }
     const int64_t values = static_cast<int64_t>(width) * height * 3;
-    auto* sse = static_cast<unsigned long long*>(scratch(context, kSlotQuantizedError, sizeof(unsigned long long)));
-    if (!sse) {
+    auto* sums = static_cast<unsigned long long*>(
+        scratch(context, kSlotQuantizedError, kEvalGroups * sizeof(unsigned long long)));
+    if (!sums) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
-    GSN_HIP(hipMemsetAsync(sse, 0, sizeof(unsigned long long), context->stream));
-    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(grid_for(values, kEvalThreads), 8192));
-    quantized_error_kernel<<<blocks, kEvalThreads, 0, context->stream>>>(image, target, quantized, values, sse);
+    const unsigned blocks = std::min(grid_for(values, 4 * kEvalThreads), kEvalGroups);
+    const bool wide = reinterpret_cast<uintptr_t>(image) % 16 == 0 && reinterpret_cast<uintptr_t>(target) % 4 == 0 &&
+                      reinterpret_cast<uintptr_t>(quantized) % 4 == 0;
+    auto* kernel = wide ? quantized_error_kernel<true> : quantized_error_kernel<false>;
+    kernel<<<blocks, kEvalThreads, 0, context->stream>>>(image, target, quantized, values, sums);
     GSN_TRY(check_launch("quantized_error_kernel"));
-    auto* host = reinterpret_cast<unsigned long long*>(static_cast<char*>(context->pinned) + 64);
-    GSN_HIP(hipMemcpyAsync(host, sse, sizeof(unsigned long long), hipMemcpyDeviceToHost, context->stream));
+    static_assert(kPinnedSums + kEvalGroups * sizeof(unsigned long long) <= kPinnedBytes, "room for the sums");
+    auto* host = reinterpret_cast<unsigned long long*>(static_cast<char*>(context->pinned) + kPinnedSums);
+    GSN_HIP(hipMemcpyAsync(host, sums, blocks * sizeof(unsigned long long), hipMemcpyDeviceToHost, context->stream));
     GSN_HIP(hipStreamSynchronize(context->stream));
-    const double total = static_cast<double>(*host);
+    unsigned long long sse = 0;
+    for (unsigned b = 0; b < blocks; ++b) {
+        sse += host[b];
+    }
+    const double total = static_cast<double>(sse);
     out[0] = total;
     out[1] = total == 0.0 ? INFINITY : -10.0 * std::log10(total / (3.0 * width * height * 255.0 * 255.0));
     return GSN_OK;

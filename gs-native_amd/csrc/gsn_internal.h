@@ -79,13 +79,17 @@ struct BackwardPrefetch {
     unsigned generation = 0;
 };
 
+// The pinned buffer: scalar readbacks below kPinnedSums, a kernel's sums from there on.
+constexpr size_t kPinnedSums = 256;
+constexpr size_t kPinnedBytes = 4096;
+
 struct gsn_context {
     hipStream_t stream = nullptr;
     int device = 0;
     int cu_count = 0;
     void* slots[kSlotCount] = {};
     size_t slot_bytes[kSlotCount] = {};
-    void* pinned = nullptr;  // small pinned host buffer for scalar readbacks
+    void* pinned = nullptr;  // small pinned host buffer for readbacks (kPinnedBytes)
     // Epoch stamp of the backward's record flags (1..127) and the flag buffer (address and size:
     // a regrown buffer may reuse the address) it was last cleared in: a byte equals the current
     // epoch (bit 7 aside) only if this step's backward reached that record.
