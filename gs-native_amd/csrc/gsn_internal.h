@@ -199,10 +199,15 @@ int exclusive_scan_int4(gsn_context* context, const Int4* input, Int4* output, i
 // (either may be the same buffer as an input only if it is not referenced by a later pass;
 // callers pass distinct buffers). keys_out may be null when only values are needed.
 // With first_histogram_ready the caller has already written the first pass's digit counts into
-// radix_histogram_buffer(context, n): entry [bin * tiles + tile] counts the elements of
-// [tile * kRadixTile, tile * kRadixTile + kRadixTile) whose low radix_first_digit_bits(bits) key
-// bits equal bin, for every bin below 1 << radix_first_digit_bits(bits).
+// radix_histogram_buffer(context, n): entry radix_table_index(bin, tile, tiles,
+// radix_table_by_tile(n)) counts the elements of [tile * kRadixTile, tile * kRadixTile + kRadixTile)
+// whose low radix_first_digit_bits(bits) key bits equal bin, for every bin below
+// 1 << radix_first_digit_bits(bits).
 constexpr int kRadixTile = 4096;
+bool radix_table_by_tile(int64_t n);
+__host__ __device__ inline int64_t radix_table_index(int bin, int tile, int tiles, bool by_tile) {
+    return by_tile ? static_cast<int64_t>(tile) * 256 + bin : static_cast<int64_t>(bin) * tiles + tile;
+}
 int* radix_histogram_buffer(gsn_context* context, int64_t n);
 int radix_first_digit_bits(int bits);
 int radix_sort_pairs(gsn_context* context, uint32_t* keys, uint32_t* values, int64_t n,

@@ -22,7 +22,7 @@ constexpr int kDepthKeyThreads = 512;
 constexpr int kDepthKeyItems = kRadixTile / kDepthKeyThreads;
 
 __global__ __launch_bounds__(kDepthKeyThreads) void depth_keys_kernel(const float* depths, const int* record_offsets,
-    uint32_t* keys, uint32_t* ids, int count, int tiles, int* histogram) {
+    uint32_t* keys, uint32_t* ids, int count, int tiles, bool by_tile, int* histogram) {
     __shared__ int s_digits[256];
     const int t = threadIdx.x;
     if (t < 256) {
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kDepthKeyThreads) void depth_keys_kernel(const floa
     }
     __syncthreads();
     if (t < 256) {
-        histogram[static_cast<int64_t>(t) * tiles + blockIdx.x] = s_digits[t];
+        histogram[radix_table_index(t, static_cast<int>(blockIdx.x), tiles, by_tile)] = s_digits[t];
     }
 }
 
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void emit_owners_kernel(const int* depth_offse
 __global__ __launch_bounds__(kEmitThreads) void emit_records_kernel(const uint32_t* __restrict__ sorted_ids,
     const int* __restrict__ depth_offsets, const int* __restrict__ owners, const int4* __restrict__ ordered_rects,
     uint32_t* __restrict__ record_tiles, uint32_t* __restrict__ record_ids, int count, int tile_count_x,
-    int record_count, int blocks, int digit_bits, int* __restrict__ histogram) {
+    int record_count, int blocks, int digit_bits, bool by_tile, int* __restrict__ histogram) {
     __shared__ int s_owner[kRadixTile];
     __shared__ int s_start[kEmitOwners];
     __shared__ uint32_t s_id[kEmitOwners];
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(kEmitThreads) void emit_records_kernel(const uint32
     }
     __syncthreads();
     if (t < (1 << digit_bits)) {
-        histogram[static_cast<int64_t>(t) * blocks + block] = s_digits[t];
+        histogram[radix_table_index(t, static_cast<int>(block), blocks, by_tile)] = s_digits[t];
     }
 }
 
@@ -371,7 +371,7 @@ int enqueue_depth_order(gsn_context* context, const float* depths, const int* re
     StageScope scope(context, kStageDepthSort);
     // 32 key bits: the first pass takes radix_first_digit_bits(32) = 8 bits, the low byte counted here.
     depth_keys_kernel<<<tiles, kDepthKeyThreads, 0, context->stream>>>(depths, record_offsets, depth_keys, depth_ids,
-        count, tiles, histogram);
+        count, tiles, radix_table_by_tile(count), histogram);
     GSN_TRY(check_launch("depth_keys_kernel"));
     return radix_sort_pairs(context, depth_keys, depth_ids, count, 32, sorted_keys, sorted_ids, true);
 }
@@ -481,7 +481,7 @@ extern "C" int gsn_build_tile_lists(gsn_context* context, const gsn_camera* came
         // kernel's arguments in range.
         emit_records_kernel<<<blocks, kEmitThreads, 0, stream>>>(sorted_ids, depth_counts, block_owners,
             ordered_rects, record_tiles, record_ids, count, camera->tile_count_x,
-            record_count, blocks, radix_first_digit_bits(tile_bits), histogram);
+            record_count, blocks, radix_first_digit_bits(tile_bits), radix_table_by_tile(record_count), histogram);
         GSN_TRY(check_launch("emit_records_kernel"));
     }
     {
