@@ -47,6 +47,10 @@ __device__ __forceinline__ void keep(float& value) {
     asm volatile("" : "+v"(value));
 }
 
+__device__ __forceinline__ void keep(int& value) {
+    asm volatile("" : "+v"(value));
+}
+
 // Calls f(state, band) for the `Bands` per-band states of a wave. Named states and not an array:
 // an array indexed by the band is moved as a whole vector register on every path.
 template<int Bands, typename State, typename F>

@@ -1,15 +1,27 @@
-// Tile keys, stable (tile, depth) ordering and per-tile ranges.
+// Per-tile Gaussian lists in depth order, without sorting the records.
 //
 // The reference (renderer.cu:223-271, 534-569) writes 64-bit keys (tile << 32 | depth bits)
 // for every record in Gaussian-id order and radix-sorts all 32 + ceil(log2 T) key bits over R
-// records. This path reaches the same order with far fewer passes over R:
-//   1. stable sort of the N visible Gaussians by depth bits (4 x 8-bit passes over N),
-//   2. records emitted in that depth order (row-major tiles inside each rectangle),
-//   3. stable sort of the records by tile id only (ceil(log2 T) bits, two passes for T <= 65536).
-// Within a tile the result is ordered by (depth bits, Gaussian id), exactly the order of a
-// stable sort of the reference keys over id-ordered records (each Gaussian has at most one
-// record per tile, and equal depth bits keep id order in both).
-#include "gsn_internal.h"
+// records. Here
+//   1. the N visible Gaussians are stably sorted by depth bits (radix_sort.hip),
+//   2. their tile rectangles are gathered in that order, once,
+//   3. the records per (chunk of the depth-ordered list, tile) are counted: a workgroup takes a chunk
+//      and a 32x32-tile part of the screen, adds the four corners of each rectangle to a difference
+//      array in LDS and sums that along both axes at the end,
+//   4. prefixes over the chunks and over the tiles give every (chunk, tile) its place in the output,
+//   5. workgroups of the same shape write the ids there, in list order.
+// Every step keeps the order of the list, so a tile's ids are ordered by (depth bits, Gaussian id):
+// exactly a stable sort of the reference keys over id-ordered records (each Gaussian has at most
+// one record per tile, and equal depth bits keep id order in both).
+// Why not a sort: a record then costs 4 bytes written, once, instead of about 48 bytes of traffic
+// through the emission of (tile, id) pairs, two radix passes over them and the search for the tiles'
+// ranges. What bounds it now: the gather of step 2 (a random line per Gaussian) and, in step 5, vector
+// instructions. Emission to ranges with the sort and so: 10K Gaussians at 256x256 45 and 25 us, 200K
+// at 979x546 88 and 79, 500K at 1248x832 160 and 123, 3M at 1920x1080 660 and 535, 2M at 3840x2160
+// 2,100 and 680.
+#include "raster_common.h"
+
+#include <algorithm>
 
 namespace gsn {
 namespace {
@@ -57,289 +69,447 @@ __global__ __launch_bounds__(kDepthKeyThreads) void depth_keys_kernel(const floa
     }
 }
 
-// Record counts and tile rectangles in depth order: the one gather by Gaussian id of the tile
-// lists. A visible Gaussian's record count is its rectangle's area; invisible Gaussians (sorted
-// last, with the key 0xffffffff that no finite depth has) get none, and their rectangles, which
-// the projection leaves unwritten, are not read.
-// One kScanBlock-entry block of [0, count] per workgroup (512 threads, eight entries each, k * 512
-// apart): the workgroup also sums its counts into block_totals[block], the first half of the
-// counts' exclusive scan.
-constexpr int kOrderThreads = 512;
-constexpr int kOrderItems = kScanBlock / kOrderThreads;
+// A part of the screen: 32x32 tiles.
+constexpr int kPartSide = 32;
+constexpr int kPartTiles = kPartSide * kPartSide;
+constexpr int kPartThreads = 1024;
 
-__global__ __launch_bounds__(kOrderThreads) void depth_order_counts_kernel(const uint32_t* sorted_ids,
-    const uint32_t* sorted_keys, const int4* tile_rects, int* counts, int4* ordered_rects, int count,
-    int* block_totals) {
-    __shared__ int s_wave_sums[kOrderThreads / 64];
-    const int t = threadIdx.x;
-    const int64_t first = static_cast<int64_t>(blockIdx.x) * kScanBlock + t;
-    int sum = 0;
+// How the screen and the list are cut. Task (chunk, part) is number chunk * parts + part.
+struct ScreenGrid {
+    int tiles_x, tiles_y;
+    int parts_x, parts;
+    int chunk, chunks;  // list entries per task
+};
+
+// A list entry's tile rectangle in 8 bytes: x0 | x1 << 16, y0 | y1 << 16 (ends exclusive).
+__device__ __forceinline__ uint2 pack_rect(int x0, int y0, int x1, int y1) {
+    return make_uint2(static_cast<uint32_t>(x0) | static_cast<uint32_t>(x1) << 16,
+        static_cast<uint32_t>(y0) | static_cast<uint32_t>(y1) << 16);
+}
+
+// Tile rectangles in depth order: the one gather by Gaussian id of the tile lists. Invisible
+// Gaussians (sorted last, with the key 0xffffffff that no finite depth has) get an empty one; their
+// rectangles, which the projection leaves unwritten, are not read. Clamped to the grid, so that
+// rectangles made for another camera cannot lead outside it.
+// Bound by the gather (16 random bytes pull a line each): several loads in flight per thread.
+constexpr int kGatherThreads = 256;
+constexpr int kGatherItems = 4;
+
+__global__ __launch_bounds__(kGatherThreads) void depth_order_rects_kernel(const uint32_t* __restrict__ sorted_ids,
+    const uint32_t* __restrict__ sorted_keys, const int4* __restrict__ tile_rects, uint2* __restrict__ rects, int count,
+    int tiles_x, int tiles_y) {
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * (kGatherThreads * kGatherItems) + threadIdx.x;
+    int4 rect[kGatherItems];
 #pragma unroll
-    for (int j = 0; j < kOrderItems; ++j) {
-        const int64_t k = first + j * kOrderThreads;
+    for (int j = 0; j < kGatherItems; ++j) {
+        const int64_t k = first + j * kGatherThreads;
+        rect[j] = make_int4(0, 0, 0, 0);
+        if (k < count && sorted_keys[k] != 0xffffffffu) {
+            rect[j] = tile_rects[min(sorted_ids[k], static_cast<uint32_t>(count - 1))];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kGatherItems; ++j) {
+        const int64_t k = first + j * kGatherThreads;
         if (k < count) {
-            int4 rect = make_int4(0, 0, 0, 0);
-            if (sorted_keys[k] != 0xffffffffu) {
-                rect = tile_rects[min(sorted_ids[k], static_cast<uint32_t>(count - 1))];
-            }
-            ordered_rects[k] = rect;
-            const int records = max(rect.z - rect.x, 0) * max(rect.w - rect.y, 0);
-            counts[k] = records;
-            sum += records;
-        }
-        else if (k == count) {
-            counts[k] = 0;
+            const int x0 = min(max(rect[j].x, 0), tiles_x), x1 = min(max(rect[j].z, 0), tiles_x);
+            const int y0 = min(max(rect[j].y, 0), tiles_y), y1 = min(max(rect[j].w, 0), tiles_y);
+            rects[k] = x1 > x0 && y1 > y0 ? pack_rect(x0, y0, x1, y1) : make_uint2(0u, 0u);
         }
     }
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
-        sum += __shfl_xor(sum, offset, 64);
+}
+
+// The chunk and part of task `number`. Tiles are numbered inside the part, 32 y + x.
+struct PartTask {
+    int64_t begin, end;  // list entries
+    int tile_x, tile_y;  // the part's first tile
+};
+
+__device__ __forceinline__ PartTask part_task(const ScreenGrid& grid, int number, int count) {
+    const int chunk = number / grid.parts;
+    const int part = number - chunk * grid.parts;
+    PartTask task;
+    task.begin = static_cast<int64_t>(chunk) * grid.chunk;
+    task.end = min(task.begin + grid.chunk, static_cast<int64_t>(count));
+    task.tile_x = part % grid.parts_x * kPartSide;
+    task.tile_y = part / grid.parts_x * kPartSide;
+    return task;
+}
+
+// A rectangle inside the part, ends in [0, 32], one byte each (x0, x1, y0, y1); false when it is
+// outside.
+__device__ __forceinline__ bool clip_to_part(uint2 rect, const PartTask& task, uint32_t& clipped) {
+    const int x0 = static_cast<int>(rect.x & 0xffff) - task.tile_x, x1 = static_cast<int>(rect.x >> 16) - task.tile_x;
+    const int y0 = static_cast<int>(rect.y & 0xffff) - task.tile_y, y1 = static_cast<int>(rect.y >> 16) - task.tile_y;
+    clipped = static_cast<uint32_t>(max(x0, 0)) | static_cast<uint32_t>(min(x1, kPartSide)) << 8 |
+              static_cast<uint32_t>(max(y0, 0)) << 16 | static_cast<uint32_t>(min(y1, kPartSide)) << 24;
+    return x0 < kPartSide && x1 > 0 && y0 < kPartSide && y1 > 0;
+}
+
+// Step 3. An entry costs about twelve instructions for the test and, where it meets the part, four
+// LDS adds, whatever its size; integer sums, so their order does not matter.
+__global__ __launch_bounds__(kPartThreads) void tile_count_kernel(const uint2* __restrict__ rects, int count,
+    ScreenGrid grid, int* __restrict__ counts) {
+    constexpr int kStride = kPartSide + 1;
+    __shared__ int s_corner[kStride * kStride];
+    for (int i = threadIdx.x; i < kStride * kStride; i += kPartThreads) {
+        s_corner[i] = 0;
     }
-    if ((t & 63) == 0) {
-        s_wave_sums[t >> 6] = sum;
+    const PartTask task = part_task(grid, static_cast<int>(blockIdx.x), count);
+    __syncthreads();
+    uint2 next = make_uint2(0u, 0u);
+    if (task.begin + threadIdx.x < task.end) {
+        next = rects[task.begin + threadIdx.x];
+    }
+    for (int64_t k = task.begin + threadIdx.x; k < task.end; k += kPartThreads) {
+        const uint2 rect = next;
+        if (k + kPartThreads < task.end) {
+            next = rects[k + kPartThreads];
+        }
+        uint32_t clipped;
+        if (clip_to_part(rect, task, clipped)) {
+            const int x0 = clipped & 0xff, x1 = (clipped >> 8) & 0xff, y0 = (clipped >> 16) & 0xff, y1 = clipped >> 24;
+            atomicAdd(&s_corner[y0 * kStride + x0], 1);
+            atomicAdd(&s_corner[y0 * kStride + x1], -1);
+            atomicAdd(&s_corner[y1 * kStride + x0], -1);
+            atomicAdd(&s_corner[y1 * kStride + x1], 1);
+        }
     }
     __syncthreads();
-    if (t == 0) {
-        int total = 0;
-#pragma unroll
-        for (int w = 0; w < kOrderThreads / 64; ++w) {
-            total += s_wave_sums[w];
+    // Running sums along x (one thread a row), then along y (one thread a column).
+    if (threadIdx.x < kPartSide) {
+        int running = 0;
+        for (int x = 0; x < kPartSide; ++x) {
+            running += s_corner[threadIdx.x * kStride + x];
+            s_corner[threadIdx.x * kStride + x] = running;
         }
-        block_totals[blockIdx.x] = total;
+    }
+    __syncthreads();
+    if (threadIdx.x < kPartSide) {
+        int running = 0;
+        for (int y = 0; y < kPartSide; ++y) {
+            running += s_corner[y * kStride + threadIdx.x];
+            s_corner[y * kStride + threadIdx.x] = running;
+        }
+    }
+    __syncthreads();
+    static_assert(kPartThreads == kPartTiles, "one tile per thread");
+    counts[static_cast<int64_t>(blockIdx.x) * kPartTiles + threadIdx.x] =
+        s_corner[(threadIdx.x / kPartSide) * kStride + threadIdx.x % kPartSide];
+}
+
+// Step 4, first half: exclusive prefixes of a part's counts over the chunks, in place, and the tiles'
+// totals. One workgroup per (part, 64 tiles): 64 tiles x 8 runs of chunks.
+__global__ __launch_bounds__(512) void tile_prefix_kernel(int* __restrict__ counts, ScreenGrid grid,
+    int* __restrict__ totals) {
+    constexpr int kRuns = 8;
+    __shared__ int s_sum[kRuns][64];
+    const int part = blockIdx.x / (kPartTiles / 64);
+    const int tile = (blockIdx.x % (kPartTiles / 64)) * 64 + (threadIdx.x & 63);
+    const int run = threadIdx.x >> 6;
+    const int rows = (grid.chunks + kRuns - 1) / kRuns;
+    const int first = min(run * rows, grid.chunks), last = min(first + rows, grid.chunks);
+    int* column = counts + static_cast<int64_t>(part) * kPartTiles + tile;
+    const int64_t stride = static_cast<int64_t>(grid.parts) * kPartTiles;
+    int sum = 0;
+#pragma unroll 8
+    for (int chunk = first; chunk < last; ++chunk) {
+        sum += column[chunk * stride];
+    }
+    s_sum[run][threadIdx.x & 63] = sum;
+    __syncthreads();
+    int running = 0, total = 0;
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+        const int value = s_sum[r][threadIdx.x & 63];
+        running += r < run ? value : 0;
+        total += value;
+    }
+#pragma unroll 8
+    for (int chunk = first; chunk < last; ++chunk) {
+        const int value = column[chunk * stride];
+        column[chunk * stride] = running;
+        running += value;
+    }
+    const int x = part % grid.parts_x * kPartSide + tile % kPartSide, y = part / grid.parts_x * kPartSide + tile / kPartSide;
+    if (run == 0 && x < grid.tiles_x && y < grid.tiles_y) {
+        totals[y * grid.tiles_x + x] = total;
     }
 }
 
-// Records are emitted in blocks of kRadixTile consecutive positions, one workgroup per block, so
-// every workgroup writes the same amount whatever the footprints (a near-camera Gaussian can own
-// thousands of records, a distant one a single record). A workgroup first needs the Gaussians
-// (in depth order) that own its positions: emit_owners_kernel stores, for every block, the
-// depth-order index of the Gaussian owning the block's first record, and in entry `blocks` the
-// owner of the last record, so block b's owners are the contiguous range [owners[b], owners[b+1]].
-constexpr int kEmitThreads = 512;
-constexpr int kEmitItems = kRadixTile / kEmitThreads;
-constexpr int kEmitOwners = kRadixTile + 1;
-
-__global__ __launch_bounds__(256) void emit_owners_kernel(const int* depth_offsets, int count, int record_count,
-    int blocks, int* owners) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) {
-        return;
-    }
-    int64_t begin = max(depth_offsets[k], 0);
-    int64_t end = min(depth_offsets[k + 1], record_count);
-    if (end <= begin) {
-        return;
-    }
-    for (int64_t b = (begin + kRadixTile - 1) / kRadixTile; b < blocks && b * kRadixTile < end; ++b) {
-        owners[b] = k;
-    }
-    if (begin <= record_count - 1 && record_count - 1 < end) {
-        owners[blocks] = k;
-    }
-}
-
-// One workgroup per block of kRadixTile records. Owner data (record start, id, rectangle) is
-// staged in LDS, every position is mapped to its owner by a max-scan over the positions where
-// owners start, and consecutive lanes then write consecutive records: (row-major tile inside the
-// owner's rectangle, Gaussian id). The workgroup also counts the low `digit_bits` bits of its
-// tile ids, which is the first pass's histogram column of the radix sort that follows (the
-// block is exactly one radix tile).
-__global__ __launch_bounds__(kEmitThreads) void emit_records_kernel(const uint32_t* __restrict__ sorted_ids,
-    const int* __restrict__ depth_offsets, const int* __restrict__ owners, const int4* __restrict__ ordered_rects,
-    uint32_t* __restrict__ record_tiles, uint32_t* __restrict__ record_ids, int count, int tile_count_x,
-    int record_count, int blocks, int digit_bits, bool by_tile, int* __restrict__ histogram) {
-    __shared__ int s_owner[kRadixTile];
-    __shared__ int s_start[kEmitOwners];
-    __shared__ uint32_t s_id[kEmitOwners];
-    __shared__ uint32_t s_corner[kEmitOwners];  // x0 | y0 << 16
-    __shared__ uint16_t s_width[kEmitOwners];
-    __shared__ int s_digits[256];
-    __shared__ int s_wave_max[kEmitThreads / 64];
-    const int t = threadIdx.x;
-    const int block = blockIdx.x;
-    const int64_t base = static_cast<int64_t>(block) * kRadixTile;
-    const int valid = static_cast<int>(min(static_cast<int64_t>(kRadixTile), record_count - base));
-    const uint32_t digit_mask = (1u << digit_bits) - 1u;
-    if (t < 256) {
-        s_digits[t] = 0;
-    }
-    const int first = min(max(owners[block], 0), count - 1);
-    const int last = min(max(owners[block + 1], first), count - 1);
-    const int owner_count = last - first + 1;
-    if (owner_count <= kEmitOwners) {
-        for (int i = t; i < kRadixTile; i += kEmitThreads) {
-            s_owner[i] = 0;
-        }
-        __syncthreads();
-        for (int o = t; o < owner_count; o += kEmitThreads) {
-            int k = first + o;
-            int start = depth_offsets[k];
-            uint32_t id = min(sorted_ids[k], static_cast<uint32_t>(count - 1));
-            int4 rect = ordered_rects[k];
-            s_start[o] = start;
-            s_id[o] = id;
-            s_corner[o] = static_cast<uint32_t>(rect.x & 0xffff) | (static_cast<uint32_t>(rect.y) << 16);
-            s_width[o] = static_cast<uint16_t>(max(rect.z - rect.x, 1));
-            int64_t position = static_cast<int64_t>(start) - base;
-            if (position < kRadixTile) {
-                // The block's first owner starts at or before the block; later owners start inside
-                // it, and of several owners starting at one position (owners without records) the
-                // last is the one whose records follow.
-                atomicMax(&s_owner[max(position, int64_t{0})], o);
-            }
-        }
-        __syncthreads();
-        // Inclusive max-scan over the positions: thread t owns positions [kEmitItems t, kEmitItems (t + 1)).
-        static_assert(kEmitItems % 4 == 0, "positions are read as int4");
-        int v[kEmitItems];
+// Step 4, second half: offsets[0 .. tiles], the exclusive prefix of the tiles' totals, by one
+// workgroup. Bound by latency: eight tiles a thread, the next 8,192 loaded meanwhile, and the results
+// go through LDS so that consecutive threads store consecutive entries.
+__global__ __launch_bounds__(1024) void tile_offsets_kernel(const int* __restrict__ totals, int tiles,
+    int64_t* __restrict__ offsets) {
+    constexpr int kItems = 8;
+    constexpr int kRound = 1024 * kItems;
+    __shared__ __align__(16) int s_out[kRound];
+    __shared__ int s_wave[16];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    auto load = [&](int64_t first, int (&values)[kItems]) {
 #pragma unroll
-        for (int q = 0; q < kEmitItems / 4; ++q) {
-            const int4 quad = *reinterpret_cast<const int4*>(&s_owner[kEmitItems * t + 4 * q]);
-            v[4 * q] = quad.x;
-            v[4 * q + 1] = quad.y;
-            v[4 * q + 2] = quad.z;
-            v[4 * q + 3] = quad.w;
+        for (int i = 0; i < kItems; ++i) {
+            values[i] = first + i < tiles ? totals[first + i] : 0;
         }
+    };
+    int carry = 0;
+    int next[kItems];
+    load(threadIdx.x * kItems, next);
+    for (int64_t base = 0; base < tiles; base += kRound) {
+        int values[kItems];
+        int sum = 0;
 #pragma unroll
-        for (int i = 1; i < kEmitItems; ++i) {
-            v[i] = max(v[i], v[i - 1]);
+        for (int i = 0; i < kItems; ++i) {
+            values[i] = next[i];
+            sum += values[i];
         }
-        const int lane = t & 63;
-        const int wave = t >> 6;
-        int scan = v[kEmitItems - 1];
+        load(base + kRound + threadIdx.x * kItems, next);
+        int inclusive = sum;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            int other = __shfl_up(scan, d, 64);
-            if (lane >= d) {
-                scan = max(scan, other);
-            }
+        for (int offset = 1; offset < 64; offset <<= 1) {
+            const int other = __shfl_up(inclusive, offset);
+            inclusive += lane >= offset ? other : 0;
         }
         if (lane == 63) {
-            s_wave_max[wave] = scan;
+            s_wave[wave] = inclusive;
         }
-        int carry = __shfl_up(scan, 1, 64);
-        if (lane == 0) {
-            carry = 0;
-        }
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) {
-            carry = max(carry, s_wave_max[w]);
+        __syncthreads();  // also ends the reads of the previous round's results
+        int running = carry + inclusive - sum;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const int total = s_wave[w];
+            running += w < wave ? total : 0;
+            carry += total;
         }
 #pragma unroll
-        for (int q = 0; q < kEmitItems / 4; ++q) {
-            *reinterpret_cast<int4*>(&s_owner[kEmitItems * t + 4 * q]) = make_int4(max(v[4 * q], carry),
-                max(v[4 * q + 1], carry), max(v[4 * q + 2], carry), max(v[4 * q + 3], carry));
+        for (int i = 0; i < kItems; ++i) {
+            s_out[threadIdx.x * kItems + i] = running;
+            running += values[i];
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kEmitItems; ++j) {
-            int p = j * kEmitThreads + t;
-            if (p < valid) {
-                int o = s_owner[p];
-                int local = static_cast<int>(base + p - s_start[o]);
-                int width = s_width[o];
-                int row = local / width;
-                int column = local - row * width;
-                uint32_t corner = s_corner[o];
-                uint32_t tile = static_cast<uint32_t>(((corner >> 16) + row) * tile_count_x + (corner & 0xffffu) + column);
-                // Written once and read once by the next sort pass: non-temporal stores keep the
-                // 240 MB of records (30M at 1080p) from displacing cached data (emit + tile sort
-                // 0.506 -> 0.473 ms).
-                __builtin_nontemporal_store(tile, record_tiles + base + p);
-                __builtin_nontemporal_store(s_id[o], record_ids + base + p);
-                atomicAdd(&s_digits[tile & digit_mask], 1);
+        for (int i = 0; i < kItems; ++i) {
+            const int64_t tile = base + i * 1024 + threadIdx.x;
+            if (tile < tiles) {
+                offsets[tile] = s_out[i * 1024 + threadIdx.x];
             }
         }
     }
-    else {
-        // Only reachable when Gaussians without records sit between ones with records (the
-        // projection never produces that): find each position's owner by binary search.
-        __syncthreads();
-        for (int j = 0; j < kEmitItems; ++j) {
-            int p = j * kEmitThreads + t;
-            if (p >= valid) {
-                continue;
-            }
-            int r = static_cast<int>(base + p);
-            int low = 0, high = count;
-            while (high - low > 1) {
-                int middle = (low + high) >> 1;
-                if (depth_offsets[middle] <= r) {
-                    low = middle;
-                }
-                else {
-                    high = middle;
-                }
-            }
-            uint32_t id = min(sorted_ids[low], static_cast<uint32_t>(count - 1));
-            int4 rect = ordered_rects[low];
-            int width = max(rect.z - rect.x, 1);
-            int local = r - depth_offsets[low];
-            int row = local / width;
-            int column = local - row * width;
-            uint32_t tile = static_cast<uint32_t>((rect.y + row) * tile_count_x + rect.x + column);
-            record_tiles[r] = tile;
-            record_ids[r] = id;
-            atomicAdd(&s_digits[tile & digit_mask], 1);
-        }
-    }
-    __syncthreads();
-    if (t < (1 << digit_bits)) {
-        histogram[radix_table_index(t, static_cast<int>(block), blocks, by_tile)] = s_digits[t];
+    if (threadIdx.x == 0) {
+        offsets[tiles] = carry;
     }
 }
 
-// Four records per thread (one 16-byte load when the run is whole): a tile's range starts at
-// the first record whose tile differs from its predecessor's.
-__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t* sorted_tiles, int64_t* offsets, int records,
-    int tile_count) {
-    const int64_t first = 4 * (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x);
-    if (first >= records) {
+// Step 5. A workgroup of 16 waves per (chunk, part). It first gathers the chunk's entries that meet
+// the part in LDS, in order (one test for the whole part instead of one per region); then each wave
+// takes an 8x8-tile region of the part and walks that list without further barriers. Entries that
+// meet the region wait in a queue until a full wave of them is there. Every tile's set of queued
+// entries is a lane mask, the AND of a row's and a column's, and the places of the region's tiles,
+// one per lane, advance by its population count.
+// What bounds it: instructions, about two thirds of them the seven per tile and queue (store_row); a
+// workgroup's busiest region, since splats of one depth crowd together and a wave lives about half of
+// its workgroup's time. Dealing out the rows of the regions evenly, with a list per region, took more
+// instructions and more time (732 against 501 us, 3M Gaussians at 1920x1080, both before the stores
+// were written out); counters in LDS and a scattered store per record 826 us; ids staged per tile in
+// LDS 1,032 us (three waves on a SIMD).
+constexpr int kListEntries = 4096;
+constexpr int kRegionSide = 8;
+constexpr int kRegions = kPartTiles / 64;  // waves of a workgroup
+
+// Row Row of the region: to each of its eight tiles, the id of the lanes in the row's and the column's
+// mask, at the address that the tile's lane holds (low, high), one id per lane below. Written out
+// because seven instructions per tile is what the kernel's time is made of (the compiler's form took
+// fourteen: a branch around the store and the address in scalar arithmetic). Addresses are read one
+// tile ahead: a store may use a scalar register five instructions after a lane read wrote it.
+template<int Row>
+__device__ __forceinline__ void store_row(int low, int high, int id, uint64_t row, const uint64_t (&column)[8]) {
+    if (row == 0) {
         return;
     }
-    int tiles[4];
-    if (first + 4 <= records) {
-        const uint4 quad = *reinterpret_cast<const uint4*>(sorted_tiles + first);
-        tiles[0] = static_cast<int>(quad.x);
-        tiles[1] = static_cast<int>(quad.y);
-        tiles[2] = static_cast<int>(quad.z);
-        tiles[3] = static_cast<int>(quad.w);
-    }
-    else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            tiles[i] = first + i < records ? static_cast<int>(sorted_tiles[first + i]) : tile_count;
+    int offset;
+#define GSN_STORE_TILE(column_mask, now, next)                          \
+    "s_and_b64 exec, %[row], " column_mask "\n"                         \
+    "v_mbcnt_lo_u32_b32 %[offset], exec_lo, 0\n"                        \
+    "v_mbcnt_hi_u32_b32 %[offset], exec_hi, %[offset]\n" next           \
+    "v_lshlrev_b32 %[offset], 2, %[offset]\n"                           \
+    "global_store_dword %[offset], %[id], s[" now "]\n"
+#define GSN_NEXT_TILE(first, second, tile) \
+    "v_readlane_b32 s" first ", %[low], " tile "\nv_readlane_b32 s" second ", %[high], " tile "\n"
+    asm volatile("s_mov_b64 s[88:89], exec\n"
+        GSN_NEXT_TILE("84", "85", "%[t0]")
+        GSN_STORE_TILE("%[c0]", "84:85", GSN_NEXT_TILE("86", "87", "%[t1]"))
+        GSN_STORE_TILE("%[c1]", "86:87", GSN_NEXT_TILE("84", "85", "%[t2]"))
+        GSN_STORE_TILE("%[c2]", "84:85", GSN_NEXT_TILE("86", "87", "%[t3]"))
+        GSN_STORE_TILE("%[c3]", "86:87", GSN_NEXT_TILE("84", "85", "%[t4]"))
+        GSN_STORE_TILE("%[c4]", "84:85", GSN_NEXT_TILE("86", "87", "%[t5]"))
+        GSN_STORE_TILE("%[c5]", "86:87", GSN_NEXT_TILE("84", "85", "%[t6]"))
+        GSN_STORE_TILE("%[c6]", "84:85", GSN_NEXT_TILE("86", "87", "%[t7]"))
+        GSN_STORE_TILE("%[c7]", "86:87", "")
+        "s_mov_b64 exec, s[88:89]"
+        : [offset] "=&v"(offset)
+        : [low] "v"(low), [high] "v"(high), [id] "v"(id), [row] "s"(row), [c0] "s"(column[0]), [c1] "s"(column[1]),
+        [c2] "s"(column[2]), [c3] "s"(column[3]), [c4] "s"(column[4]), [c5] "s"(column[5]), [c6] "s"(column[6]),
+        [c7] "s"(column[7]), [t0] "n"(8 * Row), [t1] "n"(8 * Row + 1), [t2] "n"(8 * Row + 2), [t3] "n"(8 * Row + 3),
+        [t4] "n"(8 * Row + 4), [t5] "n"(8 * Row + 5), [t6] "n"(8 * Row + 6), [t7] "n"(8 * Row + 7)
+        : "s84", "s85", "s86", "s87", "s88", "s89", "scc", "memory");
+#undef GSN_STORE_TILE
+#undef GSN_NEXT_TILE
+}
+
+__global__ __launch_bounds__(64 * kRegions) void tile_write_kernel(const uint2* __restrict__ rects,
+    const uint32_t* __restrict__ list_ids, int count, ScreenGrid grid, const int* __restrict__ prefixes,
+    const int64_t* __restrict__ offsets, int record_count, int* __restrict__ ids) {
+    __shared__ uint2 s_list[kListEntries];  // id; x0, x1, y0, y1 in the part, a byte each
+    __shared__ uint2 s_queue[kRegions][128];  // id, columns | rows << 8 in the region
+    __shared__ int s_hits[kRegions];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int number = static_cast<int>(blockIdx.x);
+    const PartTask task = part_task(grid, number, count);
+    const int region_x = wave % (kPartSide / kRegionSide) * kRegionSide;
+    const int region_y = wave / (kPartSide / kRegionSide) * kRegionSide;
+    int place = 0;  // of the lane's tile
+    {
+        const int x = region_x + lane % kRegionSide, y = region_y + lane / kRegionSide;
+        if (task.tile_x + x < grid.tiles_x && task.tile_y + y < grid.tiles_y) {
+            place = static_cast<int>(offsets[static_cast<int64_t>(task.tile_y + y) * grid.tiles_x + task.tile_x + x]) +
+                    prefixes[static_cast<int64_t>(number) * kPartTiles + y * kPartSide + x];
         }
     }
-    // Tile ids come from rectangles clamped to the grid; the clamp keeps writes inside
-    // offsets[0..T] even for rectangles produced with a different camera.
-    int previous = first == 0 ? -1 : min(max(static_cast<int>(sorted_tiles[first - 1]), 0), tile_count);
+    uint2* queue = s_queue[wave];
+    int queued = 0;
+    for (int64_t batch = task.begin; batch < task.end; batch += kListEntries) {
+        const int entries = static_cast<int>(min(task.end - batch, static_cast<int64_t>(kListEntries)));
+        // The part's list: each wave takes a run of the batch.
+        const int run = ((entries + kRegions - 1) / kRegions + 63) & ~63;
+        const int first = wave * run;
+        constexpr int kSteps = kListEntries / kRegions / 64;
+        uint32_t id[kSteps], clipped[kSteps];
+        uint64_t meets[kSteps];
+        uint2 rect[kSteps];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t r = first + i;
-        if (r >= records) {
-            break;
+        for (int j = 0; j < kSteps; ++j) {
+            const int e = first + j * 64 + lane;
+            const bool exists = j * 64 < run && e < entries;
+            rect[j] = exists ? rects[batch + e] : make_uint2(0u, 0u);
+            id[j] = exists ? list_ids[batch + e] : 0u;
         }
-        const int tile = min(max(tiles[i], 0), tile_count);
-        for (int t = previous + 1; t <= tile; ++t) {
-            offsets[t] = r;
+        int hits = 0;
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) {
+            meets[j] = lanes_where(clip_to_part(rect[j], task, clipped[j]));
+            hits += __popcll(meets[j]);
         }
-        previous = tile;
-        if (r == records - 1) {
-            for (int t = tile + 1; t <= tile_count; ++t) {
-                offsets[t] = records;
+        if (batch != task.begin) {
+            __syncthreads();  // the previous batch's list is done with
+        }
+        if (lane == 0) {
+            s_hits[wave] = hits;
+        }
+        __syncthreads();
+        int at = 0, listed = 0;
+#pragma unroll
+        for (int w = 0; w < kRegions; ++w) {
+            const int other = s_hits[w];
+            at += w < wave ? other : 0;
+            listed += other;
+        }
+        listed = __builtin_amdgcn_readfirstlane(listed);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) {
+            if (in_lanes(meets[j])) {
+                s_list[at + lanes_below(meets[j])] = make_uint2(id[j], clipped[j]);
             }
+            at += __popcll(meets[j]);
+        }
+        __syncthreads();
+        const bool last = batch + kListEntries >= task.end;
+        int base = 0;
+#pragma unroll 1
+        while (true) {
+            if (queued < 64 && base < listed) {
+                // 64 entries of the list: those that meet the region join the queue.
+                const uint2 entry = base + lane < listed ? s_list[base + lane] : make_uint2(0u, 0u);
+                base += 64;
+                const int x0 = max(static_cast<int>(entry.y & 0xff) - region_x, 0);
+                const int x1 = min(static_cast<int>(entry.y >> 8 & 0xff) - region_x, kRegionSide);
+                const int y0 = max(static_cast<int>(entry.y >> 16 & 0xff) - region_y, 0);
+                const int y1 = min(static_cast<int>(entry.y >> 24) - region_y, kRegionSide);
+                const uint64_t hit = lanes_where(x0 < x1 && y0 < y1);
+                if (in_lanes(hit)) {
+                    queue[queued + lanes_below(hit)] = make_uint2(entry.x,
+                        ((1u << x1) - (1u << x0)) | ((1u << y1) - (1u << y0)) << kRegionSide);
+                }
+                queued += __popcll(hit);
+                continue;
+            }
+            if (queued < 64 && (!last || queued == 0)) {
+                break;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const uint2 entry = lane < queued ? queue[lane] : make_uint2(0u, 0u);
+            const uint2 rest = queue[64 + lane];
+            const int id = static_cast<int>(entry.x);
+            const uint32_t columns = entry.y & 0xff, rows = entry.y >> kRegionSide;
+            uint64_t row[kRegionSide], column[kRegionSide];
+            uint64_t row_mask = 0, column_mask = 0;  // of the lane's tile
+            int tile_row = lane / kRegionSide, tile_column = lane % kRegionSide;
+            keep(tile_row);  // or the compiler keeps the 16 comparisons in registers for the whole walk
+            keep(tile_column);
+#pragma unroll
+            for (int i = 0; i < kRegionSide; ++i) {
+                row[i] = lanes_where((rows >> i & 1) != 0);
+                column[i] = lanes_where((columns >> i & 1) != 0);
+                row_mask = tile_row == i ? row[i] : row_mask;
+                column_mask = tile_column == i ? column[i] : column_mask;
+            }
+            const uint64_t mask = row_mask & column_mask;
+            const int taken = __popcll(mask);
+            // Places past the caller's record count (rectangles of another camera) are not written.
+            if (lanes_where(taken > record_count - place) != 0) {
+                queued = 0;
+                continue;
+            }
+            const uint64_t to = reinterpret_cast<uint64_t>(ids + place);
+            const int low = static_cast<int>(to), high = static_cast<int>(to >> 32);
+            store_row<0>(low, high, id, row[0], column);
+            store_row<1>(low, high, id, row[1], column);
+            store_row<2>(low, high, id, row[2], column);
+            store_row<3>(low, high, id, row[3], column);
+            store_row<4>(low, high, id, row[4], column);
+            store_row<5>(low, high, id, row[5], column);
+            store_row<6>(low, high, id, row[6], column);
+            store_row<7>(low, high, id, row[7], column);
+            place += taken;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            queue[lane] = rest;
+            queued = max(queued - 64, 0);
         }
     }
 }
 
-__global__ __launch_bounds__(256) void sorted_keys_kernel(const uint32_t* sorted_tiles, const int* ids, const float* depths,
-    uint64_t* keys, int records) {
+// The reference's sort keys of the finished lists (optional output): a record's tile is the last one
+// that begins at or before it.
+__global__ __launch_bounds__(256) void sorted_keys_kernel(const int64_t* __restrict__ offsets, int tiles,
+    const int* __restrict__ ids, const float* __restrict__ depths, uint64_t* __restrict__ keys, int records) {
     int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= records) {
         return;
     }
-    keys[r] = (static_cast<uint64_t>(sorted_tiles[r]) << 32) | float_to_bits(depths[ids[r]]);
+    int low = 0, high = tiles;
+    while (high - low > 1) {
+        const int middle = (low + high) >> 1;
+        if (offsets[middle] <= r) {
+            low = middle;
+        }
+        else {
+            high = middle;
+        }
+    }
+    keys[r] = (static_cast<uint64_t>(static_cast<uint32_t>(low)) << 32) | float_to_bits(depths[ids[r]]);
 }
 
 __global__ void zero_offsets_kernel(int64_t* offsets, int entries) {
@@ -351,14 +521,71 @@ __global__ void zero_offsets_kernel(int64_t* offsets, int entries) {
 
 } // namespace
 
+// Chunks: at least about 2,048 tasks, so that short lists still spread over the CUs (200K Gaussians at
+// 979x546, chunks of 512 and 256: writing 50 and 72 us; 500K at 1248x832, 2,048 and 4,096: 89 and 128),
+// up to 8,192 entries, where counts and prefixes have become short (2M at 3840x2160, 4,096 and 8,192:
+// counting 116 and 85 us, prefix 35 and 19, writing 546 and 519). Longer ones only where the counts
+// would exceed 65,536 tasks of 4 KB.
+static ScreenGrid screen_grid(int count, int tiles_x, int tiles_y) {
+    ScreenGrid grid{};
+    grid.tiles_x = tiles_x;
+    grid.tiles_y = tiles_y;
+    grid.parts_x = (tiles_x + kPartSide - 1) / kPartSide;
+    grid.parts = grid.parts_x * ((tiles_y + kPartSide - 1) / kPartSide);
+    const int64_t work = static_cast<int64_t>(count) * grid.parts;
+    int64_t chunk = 256;
+    while (chunk < count && ((chunk < 8192 && chunk * 2048 < work) || chunk * 65536 < work)) {
+        chunk *= 2;
+    }
+    grid.chunk = static_cast<int>(std::min<int64_t>(chunk, 1 << 30));
+    grid.chunks = static_cast<int>((static_cast<int64_t>(count) + grid.chunk - 1) / grid.chunk);
+    return grid;
+}
+
+// The lists, from the depth order: steps 2 to 5.
+static int enqueue_lists(gsn_context* context, const ScreenGrid& grid, int count, const int4* tile_rects,
+    int record_count, int* ids, int64_t* offsets) {
+    const size_t n = static_cast<size_t>(count);
+    const size_t tile_count = static_cast<size_t>(grid.tiles_x) * grid.tiles_y;
+    const int64_t tasks = static_cast<int64_t>(grid.chunks) * grid.parts;
+    const uint32_t* sorted_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedIds, n * 4));
+    const uint32_t* sorted_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedKeys, n * 4));
+    uint2* rects = static_cast<uint2*>(scratch(context, kSlotDepthRects, n * sizeof(uint2)));
+    int* counts = static_cast<int*>(scratch(context, kSlotTileCounts, static_cast<size_t>(tasks) * kPartTiles * 4));
+    int* totals = static_cast<int*>(scratch(context, kSlotTileTotals, tile_count * 4));
+    if (!sorted_ids || !sorted_keys || !rects || !counts || !totals) {
+        return GSN_ERROR_OUT_OF_MEMORY;
+    }
+    hipStream_t stream = context->stream;
+    {
+        StageScope scope(context, kStageEmit);
+        depth_order_rects_kernel<<<grid_for(count, kGatherThreads * kGatherItems), kGatherThreads, 0, stream>>>(
+            sorted_ids, sorted_keys, tile_rects, rects, count, grid.tiles_x, grid.tiles_y);
+        GSN_TRY(check_launch("depth_order_rects_kernel"));
+    }
+    {
+        StageScope scope(context, kStageRanges);
+        tile_count_kernel<<<static_cast<unsigned>(tasks), kPartThreads, 0, stream>>>(rects, count, grid, counts);
+        GSN_TRY(check_launch("tile_count_kernel"));
+        tile_prefix_kernel<<<static_cast<unsigned>(grid.parts * (kPartTiles / 64)), 512, 0, stream>>>(counts, grid, totals);
+        GSN_TRY(check_launch("tile_prefix_kernel"));
+        tile_offsets_kernel<<<1, 1024, 0, stream>>>(totals, static_cast<int>(tile_count), offsets);
+        GSN_TRY(check_launch("tile_offsets_kernel"));
+    }
+    StageScope scope(context, kStageTileSort);
+    tile_write_kernel<<<static_cast<unsigned>(tasks), 64 * kRegions, 0, stream>>>(rects, sorted_ids, count, grid,
+        counts, offsets, record_count, ids);
+    return check_launch("tile_write_kernel");
+}
+
 // Stable order of the N Gaussians by depth bits (visible ones first) into the depth-order slots:
 // sorted ids and sorted keys.
 int enqueue_depth_order(gsn_context* context, const float* depths, const int* record_offsets, int count) {
     size_t n = static_cast<size_t>(count);
-    uint32_t* depth_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthKeys, n * 4));
-    uint32_t* depth_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthIds, n * 4));
     uint32_t* sorted_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedIds, n * 4));
     uint32_t* sorted_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedKeys, n * 4));
+    uint32_t* depth_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthKeys, n * 4));
+    uint32_t* depth_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthIds, n * 4));
     if (!depth_keys || !depth_ids || !sorted_ids || !sorted_keys) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
@@ -435,8 +662,6 @@ extern "C" int gsn_build_tile_lists(gsn_context* context, const gsn_camera* came
     if (!tile_rects || !depths || !tile_gaussian_ids) {
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_build_tile_lists: null buffer");
     }
-    size_t n = static_cast<size_t>(count);
-    size_t r = static_cast<size_t>(record_count);
     const bool ordered = context->ordered_depths == depths && context->ordered_offsets == record_offsets &&
                          context->ordered_count == count;
     context->ordered_depths = nullptr;
@@ -445,64 +670,12 @@ extern "C" int gsn_build_tile_lists(gsn_context* context, const gsn_camera* came
     if (!ordered) {
         GSN_TRY(enqueue_depth_order(context, depths, record_offsets, count));
     }
-    uint32_t* sorted_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedIds, n * 4));
-    uint32_t* depth_sorted_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedKeys, n * 4));
-    int4* ordered_rects = static_cast<int4*>(scratch(context, kSlotDepthRects, n * sizeof(int4)));
-    int* depth_counts = static_cast<int*>(scratch(context, kSlotDepthCounts, (n + 1) * 4));
-    uint32_t* record_tiles = static_cast<uint32_t*>(scratch(context, kSlotRecordTiles, r * 4));
-    uint32_t* record_ids = static_cast<uint32_t*>(scratch(context, kSlotRecordIds, r * 4));
-    if (!sorted_ids || !depth_sorted_keys || !ordered_rects || !depth_counts || !record_tiles || !record_ids) {
-        return GSN_ERROR_OUT_OF_MEMORY;
-    }
-    int tile_bits = 0;
-    for (unsigned t = static_cast<unsigned>(tile_count - 1); t; t >>= 1) {
-        ++tile_bits;
-    }
-    const int blocks = static_cast<int>((static_cast<int64_t>(record_count) + kRadixTile - 1) / kRadixTile);
-    uint32_t* sorted_tiles = static_cast<uint32_t*>(scratch(context, kSlotSortKeysB, r * 4));
-    int* block_owners = static_cast<int*>(scratch(context, kSlotEmitOwners, (static_cast<size_t>(blocks) + 1) * 4));
-    int* histogram = radix_histogram_buffer(context, record_count);
-    const int count_blocks = static_cast<int>((static_cast<int64_t>(count) + kScanBlock) / kScanBlock);  // count + 1 entries
-    int* count_totals = static_cast<int*>(scratch(context, kSlotDepthCountTotals, static_cast<size_t>(count_blocks) * 4));
-    if (!sorted_tiles || !block_owners || !histogram || !count_totals) {
-        return GSN_ERROR_OUT_OF_MEMORY;
-    }
-    {
-        StageScope scope(context, kStageEmit);
-        depth_order_counts_kernel<<<count_blocks, kOrderThreads, 0, stream>>>(sorted_ids, depth_sorted_keys,
-            reinterpret_cast<const int4*>(tile_rects), depth_counts, ordered_rects, count, count_totals);
-        GSN_TRY(check_launch("depth_order_counts_kernel"));
-        GSN_TRY(exclusive_scan_int_from_totals(context, depth_counts, depth_counts, static_cast<int64_t>(count) + 1,
-            count_totals));
-        emit_owners_kernel<<<grid_for(count, 256), 256, 0, stream>>>(depth_counts, count, record_count, blocks,
-            block_owners);
-        GSN_TRY(check_launch("emit_owners_kernel"));
-        // With a single tile (tile_bits == 0) the histogram is not used; one digit bit keeps the
-        // kernel's arguments in range.
-        emit_records_kernel<<<blocks, kEmitThreads, 0, stream>>>(sorted_ids, depth_counts, block_owners,
-            ordered_rects, record_tiles, record_ids, count, camera->tile_count_x,
-            record_count, blocks, radix_first_digit_bits(tile_bits), radix_table_by_tile(record_count), histogram);
-        GSN_TRY(check_launch("emit_records_kernel"));
-    }
-    {
-        StageScope scope(context, kStageTileSort);
-        if (tile_bits == 0) {
-            GSN_HIP(hipMemcpyAsync(tile_gaussian_ids, record_ids, r * 4, hipMemcpyDeviceToDevice, stream));
-            GSN_HIP(hipMemcpyAsync(sorted_tiles, record_tiles, r * 4, hipMemcpyDeviceToDevice, stream));
-        }
-        else {
-            GSN_TRY(radix_sort_pairs(context, record_tiles, record_ids, record_count, tile_bits, sorted_tiles,
-                reinterpret_cast<uint32_t*>(tile_gaussian_ids), true));
-        }
-    }
-    // The ranges kernel writes every entry of tile_offsets[0..T] when R > 0.
-    StageScope scope(context, kStageRanges);
-    tile_ranges_kernel<<<grid_for((static_cast<int64_t>(record_count) + 3) / 4, 256), 256, 0, stream>>>(sorted_tiles,
-        tile_offsets, record_count, tile_count);
-    GSN_TRY(check_launch("tile_ranges_kernel"));
+    const ScreenGrid grid = screen_grid(count, camera->tile_count_x, camera->tile_count_y);
+    const int4* rects = reinterpret_cast<const int4*>(tile_rects);
+    GSN_TRY(enqueue_lists(context, grid, count, rects, record_count, tile_gaussian_ids, tile_offsets));
     if (sorted_keys) {
-        sorted_keys_kernel<<<grid_for(record_count, 256), 256, 0, stream>>>(sorted_tiles, tile_gaussian_ids, depths,
-            sorted_keys, record_count);
+        sorted_keys_kernel<<<grid_for(record_count, 256), 256, 0, stream>>>(tile_offsets, tile_count, tile_gaussian_ids,
+            depths, sorted_keys, record_count);
         GSN_TRY(check_launch("sorted_keys_kernel"));
     }
     return GSN_OK;
