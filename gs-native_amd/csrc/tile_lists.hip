@@ -69,6 +69,77 @@ __global__ __launch_bounds__(kDepthKeyThreads) void depth_keys_kernel(const floa
     }
 }
 
+// The depth order of few Gaussians by counting: a Gaussian's place is the number of keys before its
+// own (smaller, or equal with a smaller id). N^2 comparisons, two vector instructions for 64 of them,
+// but two launches, where the radix sort's eight to twelve dependent ones of about 5 us each set the
+// time. Lists of 4K, 10K, 16K, 20K, 24K and 32K Gaussians in all:
+// 66, 73, 73, 75, 77 and 79 us with the radix sort, 31, 40, 46, 64, 68 and 94 us so.
+constexpr int kRankCount = 24576;  // most Gaussians ordered this way
+constexpr int kRankThreads = 256;
+constexpr int kRankRun = kRankThreads;  // keys that a workgroup compares its 256 Gaussians with
+
+__device__ __forceinline__ uint32_t depth_key(const float* depths, const int* record_offsets, int i) {
+    return record_offsets[i + 1] > record_offsets[i] ? float_to_bits(depths[i]) : 0xffffffffu;
+}
+
+// Many short runs: each is a chain of LDS reads, and the chip needs a few thousand waves to hide it.
+__global__ __launch_bounds__(kRankThreads) void depth_rank_kernel(const float* __restrict__ depths,
+    const int* __restrict__ record_offsets, int count, int* __restrict__ before) {
+    __shared__ __align__(16) uint32_t s_keys[kRankRun];
+    const int i = blockIdx.x * kRankThreads + threadIdx.x;
+    const int other = blockIdx.y * kRankRun + threadIdx.x;
+    const uint32_t own = i < count ? depth_key(depths, record_offsets, i) : 0u;
+    // Past the last key: none is before another (equal ones have larger ids).
+    s_keys[threadIdx.x] = other < count ? depth_key(depths, record_offsets, other) : 0xffffffffu;
+    __syncthreads();
+    const uint4* fours = reinterpret_cast<const uint4*>(s_keys);
+    int ranked = 0;
+    if (blockIdx.y < blockIdx.x) {
+        // All ids of the run are smaller: equal keys come before.
+#pragma unroll 8
+        for (int j = 0; j < kRankRun / 4; ++j) {
+            const uint4 k = fours[j];
+            ranked += (k.x <= own) + (k.y <= own) + (k.z <= own) + (k.w <= own);
+        }
+    }
+    else if (blockIdx.y > blockIdx.x) {
+#pragma unroll 8
+        for (int j = 0; j < kRankRun / 4; ++j) {
+            const uint4 k = fours[j];
+            ranked += (k.x < own) + (k.y < own) + (k.z < own) + (k.w < own);
+        }
+    }
+    else {
+        const int self = static_cast<int>(threadIdx.x);
+#pragma unroll 8
+        for (int j = 0; j < kRankRun / 4; ++j) {
+            const uint4 k = fours[j];
+            ranked += (k.x < own) + (k.y < own) + (k.z < own) + (k.w < own);
+            ranked += (k.x == own && 4 * j < self) + (k.y == own && 4 * j + 1 < self) +
+                      (k.z == own && 4 * j + 2 < self) + (k.w == own && 4 * j + 3 < self);
+        }
+    }
+    if (i < count) {
+        before[static_cast<int64_t>(blockIdx.y) * count + i] = ranked;
+    }
+}
+
+__global__ __launch_bounds__(kRankThreads) void depth_rank_scatter_kernel(const float* __restrict__ depths,
+    const int* __restrict__ record_offsets, int count, int runs, const int* __restrict__ before,
+    uint32_t* __restrict__ sorted_keys, uint32_t* __restrict__ sorted_ids) {
+    const int i = blockIdx.x * kRankThreads + threadIdx.x;
+    if (i >= count) {
+        return;
+    }
+    int place = 0;
+#pragma unroll 16
+    for (int run = 0; run < runs; ++run) {
+        place += before[static_cast<int64_t>(run) * count + i];
+    }
+    sorted_keys[place] = depth_key(depths, record_offsets, i);
+    sorted_ids[place] = static_cast<uint32_t>(i);
+}
+
 // A part of the screen: 32x32 tiles.
 constexpr int kPartSide = 32;
 constexpr int kPartTiles = kPartSide * kPartSide;
@@ -584,6 +655,20 @@ int enqueue_depth_order(gsn_context* context, const float* depths, const int* re
     size_t n = static_cast<size_t>(count);
     uint32_t* sorted_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedIds, n * 4));
     uint32_t* sorted_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedKeys, n * 4));
+    if (count <= kRankCount) {
+        const unsigned groups = grid_for(count, kRankThreads), runs = grid_for(count, kRankRun);
+        int* before = static_cast<int*>(scratch(context, kSlotDepthKeys, n * runs * 4));
+        if (!sorted_ids || !sorted_keys || !before) {
+            return GSN_ERROR_OUT_OF_MEMORY;
+        }
+        StageScope scope(context, kStageDepthSort);
+        depth_rank_kernel<<<dim3(groups, runs), kRankThreads, 0, context->stream>>>(depths, record_offsets, count,
+            before);
+        GSN_TRY(check_launch("depth_rank_kernel"));
+        depth_rank_scatter_kernel<<<groups, kRankThreads, 0, context->stream>>>(depths, record_offsets, count,
+            static_cast<int>(runs), before, sorted_keys, sorted_ids);
+        return check_launch("depth_rank_scatter_kernel");
+    }
     uint32_t* depth_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthKeys, n * 4));
     uint32_t* depth_ids = static_cast<uint32_t*>(scratch(context, kSlotDepthIds, n * 4));
     if (!depth_keys || !depth_ids || !sorted_ids || !sorted_keys) {
