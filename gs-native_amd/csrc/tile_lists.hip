@@ -379,9 +379,11 @@ __global__ __launch_bounds__(1024) void tile_offsets_kernel(const int* __restric
 // meet the region wait in a queue until a full wave of them is there. Every tile's set of queued
 // entries is a lane mask, the AND of a row's and a column's, and the places of the region's tiles,
 // one per lane, advance by its population count.
-// What bounds it: instructions, about two thirds of them the seven per tile and queue (store_row); a
-// workgroup's busiest region, since splats of one depth crowd together and a wave lives about half of
-// its workgroup's time. Dealing out the rows of the regions evenly, with a list per region, took more
+// What bounds it: instructions, half of them the seven per tile and queue (store_row), a quarter the
+// walk of the list and a quarter the gathering (3M Gaussians at 1920x1080: 195, 85 and 92 us of 385 with
+// four-byte corners in the list and the compiler's selects, 342 in all so; without the stores
+// themselves 371); and a workgroup's busiest region, since splats of one depth crowd together. Eight
+// waves a SIMD need at most 96 scalar registers: two workgroups then fit on a CU. Dealing out the rows of the regions evenly, with a list per region, took more
 // instructions and more time (732 against 501 us, 3M Gaussians at 1920x1080, both before the stores
 // were written out); counters in LDS and a scattered store per record 826 us; ids staged per tile in
 // LDS 1,032 us (three waves on a SIMD).
@@ -389,13 +391,45 @@ constexpr int kListEntries = 4096;
 constexpr int kRegionSide = 8;
 constexpr int kRegions = kPartTiles / 64;  // waves of a workgroup
 
+// For every lane the mask of its tile's column (low, high), under one constant lane mask per column:
+// three instructions a column where a select takes six.
+__device__ __forceinline__ void column_masks(const uint64_t (&column)[8], int& low, int& high) {
+#define GSN_COLUMN(low_half, high_half, next) \
+    "v_mov_b32 %[low], " low_half "\nv_mov_b32 %[high], " high_half "\n" next
+#define GSN_NEXT_COLUMN "s_lshl_b64 exec, exec, 1\n"
+    auto half = [&](int i, int part) { return static_cast<uint32_t>(column[i] >> (32 * part)); };
+    asm volatile("s_mov_b64 s[80:81], exec\n"
+        "s_mov_b32 exec_lo, 0x01010101\n"
+        "s_mov_b32 exec_hi, 0x01010101\n"
+        GSN_COLUMN("%[l0]", "%[h0]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l1]", "%[h1]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l2]", "%[h2]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l3]", "%[h3]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l4]", "%[h4]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l5]", "%[h5]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l6]", "%[h6]", GSN_NEXT_COLUMN)
+        GSN_COLUMN("%[l7]", "%[h7]", "")
+        "s_mov_b64 exec, s[80:81]"
+        : [low] "+v"(low), [high] "+v"(high)
+        : [l0] "s"(half(0, 0)), [h0] "s"(half(0, 1)), [l1] "s"(half(1, 0)), [h1] "s"(half(1, 1)),
+        [l2] "s"(half(2, 0)), [h2] "s"(half(2, 1)), [l3] "s"(half(3, 0)), [h3] "s"(half(3, 1)),
+        [l4] "s"(half(4, 0)), [h4] "s"(half(4, 1)), [l5] "s"(half(5, 0)), [h5] "s"(half(5, 1)),
+        [l6] "s"(half(6, 0)), [h6] "s"(half(6, 1)), [l7] "s"(half(7, 0)), [h7] "s"(half(7, 1))
+        : "s80", "s81", "scc");
+#undef GSN_COLUMN
+#undef GSN_NEXT_COLUMN
+}
+
 // Row Row of the region: to each of its eight tiles, the id of the lanes in the row's and the column's
-// mask, at the address that the tile's lane holds (low, high), one id per lane below. Written out
-// because seven instructions per tile is what the kernel's time is made of (the compiler's form took
-// fourteen: a branch around the store and the address in scalar arithmetic). Addresses are read one
-// tile ahead: a store may use a scalar register five instructions after a lane read wrote it.
+// mask, at the address that the tile's lane holds (low, high), one id per lane below; the row's mask
+// to its tiles' lanes. Written out because seven instructions per tile is what the kernel's time is
+// made of (the compiler's form took fourteen: a branch around the store and the address in scalar
+// arithmetic). Addresses are read one tile ahead: a store may use a scalar register five instructions
+// after a lane read wrote it.
 template<int Row>
-__device__ __forceinline__ void store_row(int low, int high, int id, uint64_t row, const uint64_t (&column)[8]) {
+__device__ __forceinline__ void store_row(int low, int high, int id, uint32_t rows, const uint64_t (&column)[8],
+    int& row_low, int& row_high) {
+    const uint64_t row = lanes_where((rows >> Row & 1) != 0);
     if (row == 0) {
         return;
     }
@@ -408,31 +442,38 @@ __device__ __forceinline__ void store_row(int low, int high, int id, uint64_t ro
     "global_store_dword %[offset], %[id], s[" now "]\n"
 #define GSN_NEXT_TILE(first, second, tile) \
     "v_readlane_b32 s" first ", %[low], " tile "\nv_readlane_b32 s" second ", %[high], " tile "\n"
-    asm volatile("s_mov_b64 s[88:89], exec\n"
-        GSN_NEXT_TILE("84", "85", "%[t0]")
-        GSN_STORE_TILE("%[c0]", "84:85", GSN_NEXT_TILE("86", "87", "%[t1]"))
-        GSN_STORE_TILE("%[c1]", "86:87", GSN_NEXT_TILE("84", "85", "%[t2]"))
-        GSN_STORE_TILE("%[c2]", "84:85", GSN_NEXT_TILE("86", "87", "%[t3]"))
-        GSN_STORE_TILE("%[c3]", "86:87", GSN_NEXT_TILE("84", "85", "%[t4]"))
-        GSN_STORE_TILE("%[c4]", "84:85", GSN_NEXT_TILE("86", "87", "%[t5]"))
-        GSN_STORE_TILE("%[c5]", "86:87", GSN_NEXT_TILE("84", "85", "%[t6]"))
-        GSN_STORE_TILE("%[c6]", "84:85", GSN_NEXT_TILE("86", "87", "%[t7]"))
-        GSN_STORE_TILE("%[c7]", "86:87", "")
-        "s_mov_b64 exec, s[88:89]"
-        : [offset] "=&v"(offset)
+    asm volatile("s_mov_b64 s[80:81], exec\n"
+        "s_mov_b32 exec_lo, %[lanes_low]\n"
+        "s_mov_b32 exec_hi, %[lanes_high]\n"
+        "v_mov_b32 %[row_low], %[mask_low]\n"
+        "v_mov_b32 %[row_high], %[mask_high]\n"
+        GSN_NEXT_TILE("76", "77", "%[t0]")
+        GSN_STORE_TILE("%[c0]", "76:77", GSN_NEXT_TILE("78", "79", "%[t1]"))
+        GSN_STORE_TILE("%[c1]", "78:79", GSN_NEXT_TILE("76", "77", "%[t2]"))
+        GSN_STORE_TILE("%[c2]", "76:77", GSN_NEXT_TILE("78", "79", "%[t3]"))
+        GSN_STORE_TILE("%[c3]", "78:79", GSN_NEXT_TILE("76", "77", "%[t4]"))
+        GSN_STORE_TILE("%[c4]", "76:77", GSN_NEXT_TILE("78", "79", "%[t5]"))
+        GSN_STORE_TILE("%[c5]", "78:79", GSN_NEXT_TILE("76", "77", "%[t6]"))
+        GSN_STORE_TILE("%[c6]", "76:77", GSN_NEXT_TILE("78", "79", "%[t7]"))
+        GSN_STORE_TILE("%[c7]", "78:79", "")
+        "s_mov_b64 exec, s[80:81]"
+        : [offset] "=&v"(offset), [row_low] "+&v"(row_low), [row_high] "+&v"(row_high)
         : [low] "v"(low), [high] "v"(high), [id] "v"(id), [row] "s"(row), [c0] "s"(column[0]), [c1] "s"(column[1]),
         [c2] "s"(column[2]), [c3] "s"(column[3]), [c4] "s"(column[4]), [c5] "s"(column[5]), [c6] "s"(column[6]),
-        [c7] "s"(column[7]), [t0] "n"(8 * Row), [t1] "n"(8 * Row + 1), [t2] "n"(8 * Row + 2), [t3] "n"(8 * Row + 3),
+        [c7] "s"(column[7]), [mask_low] "s"(static_cast<uint32_t>(row)), [mask_high] "s"(static_cast<uint32_t>(row >> 32)),
+        [lanes_low] "n"(Row < 4 ? 0xff << (8 * (Row & 3)) : 0), [lanes_high] "n"(Row < 4 ? 0 : 0xff << (8 * (Row & 3))),
+        [t0] "n"(8 * Row), [t1] "n"(8 * Row + 1), [t2] "n"(8 * Row + 2), [t3] "n"(8 * Row + 3),
         [t4] "n"(8 * Row + 4), [t5] "n"(8 * Row + 5), [t6] "n"(8 * Row + 6), [t7] "n"(8 * Row + 7)
-        : "s84", "s85", "s86", "s87", "s88", "s89", "scc", "memory");
+        : "s76", "s77", "s78", "s79", "s80", "s81", "scc", "memory");
 #undef GSN_STORE_TILE
 #undef GSN_NEXT_TILE
 }
 
-__global__ __launch_bounds__(64 * kRegions) void tile_write_kernel(const uint2* __restrict__ rects,
+__global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint2* __restrict__ rects,
     const uint32_t* __restrict__ list_ids, int count, ScreenGrid grid, const int* __restrict__ prefixes,
     const int64_t* __restrict__ offsets, int record_count, int* __restrict__ ids) {
-    __shared__ uint2 s_list[kListEntries];  // id; x0, x1, y0, y1 in the part, a byte each
+    __shared__ uint32_t s_id[kListEntries];
+    __shared__ uint2 s_bits[kListEntries];  // columns and rows of the part, a bit each
     __shared__ uint2 s_queue[kRegions][128];  // id, columns | rows << 8 in the region
     __shared__ int s_hits[kRegions];
     const int lane = threadIdx.x & 63;
@@ -442,13 +483,17 @@ __global__ __launch_bounds__(64 * kRegions) void tile_write_kernel(const uint2* 
     const int region_x = wave % (kPartSide / kRegionSide) * kRegionSide;
     const int region_y = wave / (kPartSide / kRegionSide) * kRegionSide;
     int place = 0;  // of the lane's tile
+    bool fits = true;
     {
         const int x = region_x + lane % kRegionSide, y = region_y + lane / kRegionSide;
         if (task.tile_x + x < grid.tiles_x && task.tile_y + y < grid.tiles_y) {
-            place = static_cast<int>(offsets[static_cast<int64_t>(task.tile_y + y) * grid.tiles_x + task.tile_x + x]) +
-                    prefixes[static_cast<int64_t>(number) * kPartTiles + y * kPartSide + x];
+            const int64_t* begin = offsets + static_cast<int64_t>(task.tile_y + y) * grid.tiles_x + task.tile_x + x;
+            place = static_cast<int>(begin[0]) + prefixes[static_cast<int64_t>(number) * kPartTiles + y * kPartSide + x];
+            fits = begin[1] <= record_count;
         }
     }
+    // A region with lists past the caller's record count (rectangles of another camera) is not written.
+    const bool writes = lanes_where(!fits) == 0;
     uint2* queue = s_queue[wave];
     int queued = 0;
     for (int64_t batch = task.begin; batch < task.end; batch += kListEntries) {
@@ -480,81 +525,81 @@ __global__ __launch_bounds__(64 * kRegions) void tile_write_kernel(const uint2* 
             s_hits[wave] = hits;
         }
         __syncthreads();
-        int at = 0, listed = 0;
-#pragma unroll
-        for (int w = 0; w < kRegions; ++w) {
-            const int other = s_hits[w];
-            at += w < wave ? other : 0;
-            listed += other;
-        }
-        listed = __builtin_amdgcn_readfirstlane(listed);
-        at = __builtin_amdgcn_readfirstlane(at);
+        // Prefix over the waves, in the lanes of a row of sixteen.
+        static_assert(kRegions == 16, "a wave's total per lane of a row");
+        int hits_to = s_hits[lane & 15];
+        hits_to += __builtin_amdgcn_update_dpp(0, hits_to, 0x111, 0xf, 0xf, true);  // row_shr:1
+        hits_to += __builtin_amdgcn_update_dpp(0, hits_to, 0x112, 0xf, 0xf, true);
+        hits_to += __builtin_amdgcn_update_dpp(0, hits_to, 0x114, 0xf, 0xf, true);
+        hits_to += __builtin_amdgcn_update_dpp(0, hits_to, 0x118, 0xf, 0xf, true);
+        const int listed = readlane_i(hits_to, 15);
+        int at = readlane_i(hits_to, wave) - hits;
 #pragma unroll
         for (int j = 0; j < kSteps; ++j) {
             if (in_lanes(meets[j])) {
-                s_list[at + lanes_below(meets[j])] = make_uint2(id[j], clipped[j]);
+                const int place_in_list = at + lanes_below(meets[j]);
+                const uint32_t x0 = clipped[j] & 0xff, x1 = clipped[j] >> 8 & 0xff;
+                const uint32_t y0 = clipped[j] >> 16 & 0xff, y1 = clipped[j] >> 24;
+                s_id[place_in_list] = id[j];
+                s_bits[place_in_list] = make_uint2(~0u >> (32 - (x1 - x0)) << x0, ~0u >> (32 - (y1 - y0)) << y0);
             }
             at += __popcll(meets[j]);
         }
         __syncthreads();
         const bool last = batch + kListEntries >= task.end;
         int base = 0;
+        uint2 next_bits = lane < listed ? s_bits[lane] : make_uint2(0u, 0u);
+        uint32_t next_id = s_id[lane];
 #pragma unroll 1
         while (true) {
-            if (queued < 64 && base < listed) {
-                // 64 entries of the list: those that meet the region join the queue.
-                const uint2 entry = base + lane < listed ? s_list[base + lane] : make_uint2(0u, 0u);
+            // 64 entries of the list at a time: those that meet the region join the queue.
+#pragma unroll 1
+            while (queued < 64 && base < listed) {
+                const uint32_t columns = next_bits.x >> region_x & 0xff, rows = next_bits.y >> region_y & 0xff;
+                const uint32_t entry_id = next_id;
                 base += 64;
-                const int x0 = max(static_cast<int>(entry.y & 0xff) - region_x, 0);
-                const int x1 = min(static_cast<int>(entry.y >> 8 & 0xff) - region_x, kRegionSide);
-                const int y0 = max(static_cast<int>(entry.y >> 16 & 0xff) - region_y, 0);
-                const int y1 = min(static_cast<int>(entry.y >> 24) - region_y, kRegionSide);
-                const uint64_t hit = lanes_where(x0 < x1 && y0 < y1);
+                const int e = min(base + lane, kListEntries - 1);
+                next_bits = s_bits[e];
+                next_id = s_id[e];
+                if (base + lane >= listed) {
+                    next_bits.x = 0;
+                }
+                const uint64_t hit = lanes_where(columns != 0) & lanes_where(rows != 0);
                 if (in_lanes(hit)) {
-                    queue[queued + lanes_below(hit)] = make_uint2(entry.x,
-                        ((1u << x1) - (1u << x0)) | ((1u << y1) - (1u << y0)) << kRegionSide);
+                    queue[queued + lanes_below(hit)] = make_uint2(entry_id, columns | rows << kRegionSide);
                 }
                 queued += __popcll(hit);
-                continue;
             }
             if (queued < 64 && (!last || queued == 0)) {
                 break;
+            }
+            if (!writes) {
+                queued = 0;
+                continue;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             const uint2 entry = lane < queued ? queue[lane] : make_uint2(0u, 0u);
             const uint2 rest = queue[64 + lane];
             const int id = static_cast<int>(entry.x);
             const uint32_t columns = entry.y & 0xff, rows = entry.y >> kRegionSide;
-            uint64_t row[kRegionSide], column[kRegionSide];
-            uint64_t row_mask = 0, column_mask = 0;  // of the lane's tile
-            int tile_row = lane / kRegionSide, tile_column = lane % kRegionSide;
-            keep(tile_row);  // or the compiler keeps the 16 comparisons in registers for the whole walk
-            keep(tile_column);
+            uint64_t column[kRegionSide];
 #pragma unroll
             for (int i = 0; i < kRegionSide; ++i) {
-                row[i] = lanes_where((rows >> i & 1) != 0);
                 column[i] = lanes_where((columns >> i & 1) != 0);
-                row_mask = tile_row == i ? row[i] : row_mask;
-                column_mask = tile_column == i ? column[i] : column_mask;
             }
-            const uint64_t mask = row_mask & column_mask;
-            const int taken = __popcll(mask);
-            // Places past the caller's record count (rectangles of another camera) are not written.
-            if (lanes_where(taken > record_count - place) != 0) {
-                queued = 0;
-                continue;
-            }
+            int row_low = 0, row_high = 0, column_low = 0, column_high = 0;  // the masks of the lane's tile
+            column_masks(column, column_low, column_high);
             const uint64_t to = reinterpret_cast<uint64_t>(ids + place);
             const int low = static_cast<int>(to), high = static_cast<int>(to >> 32);
-            store_row<0>(low, high, id, row[0], column);
-            store_row<1>(low, high, id, row[1], column);
-            store_row<2>(low, high, id, row[2], column);
-            store_row<3>(low, high, id, row[3], column);
-            store_row<4>(low, high, id, row[4], column);
-            store_row<5>(low, high, id, row[5], column);
-            store_row<6>(low, high, id, row[6], column);
-            store_row<7>(low, high, id, row[7], column);
-            place += taken;
+            store_row<0>(low, high, id, rows, column, row_low, row_high);
+            store_row<1>(low, high, id, rows, column, row_low, row_high);
+            store_row<2>(low, high, id, rows, column, row_low, row_high);
+            store_row<3>(low, high, id, rows, column, row_low, row_high);
+            store_row<4>(low, high, id, rows, column, row_low, row_high);
+            store_row<5>(low, high, id, rows, column, row_low, row_high);
+            store_row<6>(low, high, id, rows, column, row_low, row_high);
+            store_row<7>(low, high, id, rows, column, row_low, row_high);
+            place += __popc(static_cast<uint32_t>(row_low & column_low)) + __popc(static_cast<uint32_t>(row_high & column_high));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             queue[lane] = rest;
             queued = max(queued - 64, 0);
