@@ -219,15 +219,16 @@ __global__ __launch_bounds__(256) void density_write_kernel(const float* __restr
         }
     }
     // The rows, kWriteRows at a time: a group's loads are all issued before its stores, and a
-    // Gaussian's row is read once for both of its outputs. 500K Gaussians:
-    // 124 us row by row and output by output, 84 us so.
+    // Gaussian's row is read once for both of its outputs. 500K Gaussians: 124 us row by row and output
+    // by output, 84 us so, 75 with non-temporal loads and the history's copy beside it non-temporal too
+    // (non-temporal stores, at places that fill no line at once: 141).
 #pragma unroll
     for (int base = 0; base < kParamCount; base += kWriteRows) {
         float values[kWriteRows];
 #pragma unroll
         for (int k = 0; k < kWriteRows; ++k) {
             if (base + k < kParamCount) {
-                values[k] = params[(base + k) * n + id];
+                values[k] = __builtin_nontemporal_load(params + (base + k) * n + id);
             }
         }
 #pragma unroll

@@ -645,6 +645,8 @@ __global__ __launch_bounds__(256) void adam_kernel(const float* __restrict__ gra
 // One thread per new Gaussian: its parent id is read once and its 58 moment pairs are gathered
 // kRemapRows rows at a time (all loads of a group in flight); neighbouring new ids mostly have
 // neighbouring parents, so each row's gathers and stores stay within one or two 512-byte pieces.
+// Bound by memory; both sides are read or written once and larger than the caches: non-temporal
+// (500K Gaussians: 126 -> 111 us, the parameters' copy beside it 84 -> 79).
 constexpr int kRemapRows = 8;
 
 __global__ __launch_bounds__(256) void remap_history_kernel(const int* parent_ids, const float* previous, float* moments,
@@ -657,20 +659,20 @@ __global__ __launch_bounds__(256) void remap_history_kernel(const int* parent_id
     const bool inherited = parent >= 0 && parent < previous_count;
 #pragma unroll
     for (int base = 0; base < kParamCount; base += kRemapRows) {
-        float2 pairs[kRemapRows];
+        moment_pair pairs[kRemapRows];
 #pragma unroll
         for (int k = 0; k < kRemapRows; ++k) {
             const int row = base + k;
-            pairs[k] = make_float2(0.0f, 0.0f);
+            pairs[k] = moment_pair{0.0f, 0.0f};
             if (row < kParamCount && inherited) {
-                pairs[k] = *reinterpret_cast<const float2*>(previous + moment_index(parent, row));
+                pairs[k] = load_moments(previous, moment_index(parent, row));
             }
         }
 #pragma unroll
         for (int k = 0; k < kRemapRows; ++k) {
             const int row = base + k;
             if (row < kParamCount) {
-                *reinterpret_cast<float2*>(moments + moment_index(id, row)) = pairs[k];
+                store_moments(moments, moment_index(id, row), pairs[k].x, pairs[k].y);
             }
         }
     }
