@@ -117,7 +117,9 @@ __global__ __launch_bounds__(kSortThreads) void radix_digit_scan_kernel(int* his
 // Fused: the table has a row per tile, and each workgroup forms its digits' starts itself: 256 digits
 // times two halves of the tiles, one coalesced row a load. For up to kFusedTiles tiles that is a few
 // memory latencies, less than a launch of radix_digit_scan_kernel (4.6 us and the gap before it).
-// 49 tiles (200,000 pairs): the scatter goes from 9.2 to 10.3 us; 123 tiles: from 10.9 to 14.6.
+// 49 tiles (200,000 pairs): the scatter went from 9.2 to 10.3 us; 123 tiles: from 10.9 to 14.6. Counting
+// the next pass's digits here too, with atomics by destination, took 70 us on depth keys (their high
+// bytes are few) and was left out.
 template<bool Fused>
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint32_t* keys_in, const uint32_t* values_in,
     int64_t n, int shift, int bits, int tiles, const int* offsets, const int* totals, uint32_t* keys_out,
@@ -127,8 +129,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
     __shared__ int s_wave_count[kWaves][256];
     __shared__ int s_digit_start[256];
     __shared__ int s_global[256];
-    __shared__ int s_scan[256];
-    __shared__ int s_base[256];
+    __shared__ int s_sums[2][4];
     __shared__ int s_half[Fused ? 2 : 1][Fused ? 256 : 1];
 
     const int t = threadIdx.x;
@@ -192,8 +193,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
         // Out-of-range slots take the largest digit so that they rank after every valid element.
         uint32_t digit = in_range ? ((key >> shift) & mask) : mask;
         uint64_t peers = ~0ull;
-        for (int b = 0; b < bits; ++b) {
-            uint64_t vote = __ballot((digit >> b) & 1u);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            // Bits past the digit's are zero in every lane and keep all peers.
+            const uint64_t vote = __ballot((digit >> b) & 1u);
             peers &= ((digit >> b) & 1u) ? vote : ~vote;
         }
         int before = __popcll(peers & lanemask_lt);
@@ -222,27 +225,31 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
         row_total = Fused ? fused_total + s_half[Fused ? 1 : 0][Fused ? t : 0] : totals[t];
         s_global[t] = Fused ? fused_before + s_half[0][Fused ? t : 0] : offsets[static_cast<int64_t>(t) * tiles + blockIdx.x];
     }
-    if (t < 256) {
-        s_scan[t] = digit_total;
-        s_base[t] = row_total;
+    // Inclusive scans over the digits of the in-tile counts and of the row totals, by four waves. (In
+    // LDS with two barriers a step, and with the votes above in a loop over `bits`, a pass took 10.2,
+    // 14.5 and 19.5 us at 49, 123 and 733 tiles; 8.5, 12.8 and 17.7 so.)
+    int digits_to = digit_total, rows_to = row_total;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+        const int digits_below = __shfl_up(digits_to, offset);
+        const int rows_below = __shfl_up(rows_to, offset);
+        digits_to += lane >= offset ? digits_below : 0;
+        rows_to += lane >= offset ? rows_below : 0;
+    }
+    if (wave < 4 && lane == 63) {
+        s_sums[0][wave] = digits_to;
+        s_sums[1][wave] = rows_to;
     }
     __syncthreads();
-    // Inclusive scans over the digits of the in-tile counts and of the row totals.
-    for (int offset = 1; offset < 256; offset <<= 1) {
-        int other = (t < 256 && t >= offset) ? s_scan[t - offset] : 0;
-        int other_base = (t < 256 && t >= offset) ? s_base[t - offset] : 0;
-        __syncthreads();
-        if (t < 256) {
-            s_scan[t] += other;
-            s_base[t] += other_base;
-        }
-        __syncthreads();
-    }
     if (t < 256) {
-        s_digit_start[t] = s_scan[t] - digit_total;
-    }
-    if (t < bins) {
-        s_global[t] += s_base[t] - row_total;
+        for (int w = 0; w < wave; ++w) {
+            digits_to += s_sums[0][w];
+            rows_to += s_sums[1][w];
+        }
+        s_digit_start[t] = digits_to - digit_total;
+        if (t < bins) {
+            s_global[t] += rows_to - row_total;
+        }
     }
     __syncthreads();
 
