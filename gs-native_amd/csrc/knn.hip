@@ -13,8 +13,8 @@
 // the waves of a SIMD. One thread per point with a stack of its own took the same walk with a
 // different node in every lane and its stack in scratch memory; a wave walking for 64 points at once
 // tested nearly every block, since the sparsest of its points set the reach of all. 200,000 points
-// of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 328 (so); about 40
-// nodes and leaves a point. The bounds of the points, reduced by every workgroup at once, 32 and 5 us.
+// of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 317 (so); about 40
+// nodes and leaves a point. Letting the searches of a wave wait for each other at their leaves took 389. The bounds of the points, reduced by every workgroup at once, 32 and 5 us.
 // Candidates are ordered by (squared distance, original index), so the three neighbours are
 // unique even with duplicate points and equal the exhaustive search with the same tie rule.
 // Squared distances are (dx*dx + dy*dy) + dz*dz with FP contraction off, as in the host
@@ -254,7 +254,9 @@ struct Waiting {
 constexpr int kNodeBits = 28;
 // The root's children and then seven a level can wait at once.
 constexpr int kStack = kFan * kMaxLevels;
-constexpr int kQueryWaves = 4;
+// Waves of a workgroup, which ends with its longest search: 328 us with four, 317 with two, 318 with
+// one (200,000 points).
+constexpr int kQueryWaves = 2;
 
 // The value of another lane of the aligned eight: across pairs, across halves of four (mirrored) or
 // the other four (mirrored).
