@@ -82,9 +82,10 @@ def log(message: str) -> None:
 def algorithmic_bytes(*, n: float, v: float, r: float, p: int, t: int, k: int = 16) -> dict:
     """Compulsory HBM bytes of one launch of each stage of this build, from its inputs and outputs:
     n Gaussians, v visible, r (tile, Gaussian) records, p pixels, t tiles, k SH coefficients per
-    channel. Sort stages count one read and one write of their (key, id) pairs (the sort's lower
-    bound; an LSD pass moves about that much again per pass). The tile records are 8 bytes (tile id,
-    Gaussian id). The per-Gaussian gradient pass with Adam fused in never writes or re-reads a
+    channel. The depth sort counts one read and one write of its (key, id) pairs (the sort's lower
+    bound; an LSD pass moves about that much again per pass). The lists: rectangles gathered in depth
+    order as 8 bytes each ("emit"), read once to count ("ranges") and once, with the ids, to write the
+    four-byte records ("tile_sort"). The per-Gaussian gradient pass with Adam fused in never writes or re-reads a
     gradient buffer: its floor is the Adam rows (params, both moments) read and written (1392n), the
     statistics written (16n), the run offsets (4n) and one flag byte per record (r); the reached
     records' 48-byte partials come on top (data-dependent, not counted)."""
@@ -92,9 +93,9 @@ def algorithmic_bytes(*, n: float, v: float, r: float, p: int, t: int, k: int = 
         "project": 16 * n + v * (28 + 12 * k + 56),
         "scan": 8 * n,
         "depth_sort": 16 * n,
-        "emit": 24 * v + 8 * r,
-        "tile_sort": 16 * r,
-        "ranges": 4 * r + 8 * (t + 1),
+        "emit": 16 * n + 16 * v,
+        "tile_sort": 12 * n + 4 * r,
+        "ranges": 8 * n + 8 * (t + 1),
         "raster_forward": 40 * r + 12 * p + 8 * (t + 1),
         "image_gradients": 27 * p,
         "raster_backward": 40 * r + 24 * p + 44 * v,

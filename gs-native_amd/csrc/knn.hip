@@ -14,7 +14,8 @@
 // different node in every lane and its stack in scratch memory; a wave walking for 64 points at once
 // tested nearly every block, since the sparsest of its points set the reach of all. 200,000 points
 // of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 317 (so); about 40
-// nodes and leaves a point. Letting the searches of a wave wait for each other at their leaves took 389. The bounds of the points, reduced by every workgroup at once, 32 and 5 us.
+// nodes and leaves a point. Letting the searches of a wave wait for each other at their leaves took
+// 389. The bounds of the points, reduced by one thread per workgroup 32 us, by all 5.
 // Candidates are ordered by (squared distance, original index), so the three neighbours are
 // unique even with duplicate points and equal the exhaustive search with the same tie rule.
 // Squared distances are (dx*dx + dy*dy) + dz*dz with FP contraction off, as in the host

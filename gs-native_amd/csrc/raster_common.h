@@ -1,10 +1,10 @@
 // Shared pieces of the tile rasteriser forward and backward kernels.
 //
-// Work decomposition (gfx950, wave64): one 64-lane workgroup per 16x16 tile. Lane l owns pixel
-// column l % 16 and, in each of four 4-row bands b = 0..3, the pixel at row 4*b + l / 16. A
-// batch of 64 records is loaded one per lane; the per-splat values are then broadcast to the
-// wave with v_readlane (scalar operands, no LDS round trip and no workgroup barrier). For each
-// splat a 4-bit band mask marks the bands its alpha >= 1/255 ellipse can reach, so whole bands
+// Work decomposition (gfx950, wave64): a 16x16 tile has four 4-row bands, of which a wave owns one,
+// two or four. Lane l owns pixel column l % 16 and, in each of the wave's bands b, the pixel at row
+// 4*b + l / 16. A batch of 64 records is loaded one per lane and those that can reach the wave's
+// bands go to a list in LDS, whose entries every lane then reads (broadcasts). For each splat a
+// 4-bit band mask marks the bands its alpha >= 1/255 ellipse can reach, so whole bands
 // are skipped with a uniform branch. The mask is conservative (margins below), so every skipped
 // (pixel, splat) pair is one the per-pixel test would have rejected anyway: results are identical
 // to evaluating every pair.

@@ -10,9 +10,9 @@
 
 #include <mutex>
 
-// Per-block sums (3 doubles per 32x16-pixel block and channel) of the largest image accepted:
+// Per-block sums (3 doubles per 32x32-pixel block and channel) of the largest image accepted:
 // 131,072 blocks = 3 MiB of device memory held on each device the library runs on, enough for
-// about 22 million pixels (e.g. 5187 x 3361).
+// about 44 million pixels.
 constexpr int64_t kStaticMetricBlocks = 131072;
 static __device__ __align__(256) double scratch[kStaticMetricBlocks * 3];
 

@@ -17,8 +17,8 @@
 // through the emission of (tile, id) pairs, two radix passes over them and the search for the tiles'
 // ranges. What bounds it now: the gather of step 2 (a random line per Gaussian) and, in step 5, vector
 // instructions. Emission to ranges with the sort and so: 10K Gaussians at 256x256 45 and 25 us, 200K
-// at 979x546 88 and 79, 500K at 1248x832 160 and 123, 3M at 1920x1080 660 and 535, 2M at 3840x2160
-// 2,100 and 680.
+// at 979x546 88 and 73, 500K at 1248x832 160 and 113, 3M at 1920x1080 660 and 494, 2M at 3840x2160
+// 2,100 and 640.
 #include "raster_common.h"
 
 #include <algorithm>
@@ -638,10 +638,11 @@ __global__ void zero_offsets_kernel(int64_t* offsets, int entries) {
 } // namespace
 
 // Chunks: at least about 2,048 tasks, so that short lists still spread over the CUs (200K Gaussians at
-// 979x546, chunks of 512 and 256: writing 50 and 72 us; 500K at 1248x832, 2,048 and 4,096: 89 and 128),
-// up to 8,192 entries, where counts and prefixes have become short (2M at 3840x2160, 4,096 and 8,192:
-// counting 116 and 85 us, prefix 35 and 19, writing 546 and 519). Longer ones only where the counts
-// would exceed 65,536 tasks of 4 KB.
+// 979x546, chunks of 512 and 256: writing 50 and 70 us, counting 9 and 16; 500K at 1248x832, 2,048 and
+// 1,024: writing 88 and 87, counting and prefixes 19 and 29), up to 8,192 entries, where counts and
+// prefixes have become short (2M at 3840x2160, 4,096, 8,192 and 16,384: all three kernels 690, 623 and
+// 654 us; 3M at 1920x1080: 459, 473 and 562). Longer ones only where the counts would exceed 65,536
+// tasks of 4 KB.
 static ScreenGrid screen_grid(int count, int tiles_x, int tiles_y) {
     ScreenGrid grid{};
     grid.tiles_x = tiles_x;

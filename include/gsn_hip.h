@@ -85,7 +85,8 @@ int gsn_device_memory_info(size_t* free_bytes, size_t* total_bytes);
  * cv::TickMeter). While enabled, every stage records a HIP event pair on the context stream;
  * gsn_context_stage_times synchronises, returns the summed milliseconds and the number of timed
  * launches of each stage, and clears the record. Stage order:
- *   0 project, 1 scan, 2 depth sort, 3 record emit, 4 tile sort, 5 tile ranges,
+ *   0 project, 1 scan, 2 depth sort, 3 rectangles in depth order, 4 tile lists' ids written,
+ *   5 tile counts and offsets,
  *   6 raster forward, 7 image gradients, 8 raster backward, 9 per-Gaussian gradients (+Adam),
  *   10 Adam, 11 density control (count, write, history remap, opacity cap), 12 KNN,
  *   13 statistics accumulation (per-view density and feature accumulators). */
@@ -164,7 +165,7 @@ int gsn_project_gaussians(gsn_context* context, const float* params, int count,
 int gsn_scan_record_offsets(gsn_context* context, int* record_offsets, int count,
     int* record_count);
 
-/* Tile keys, stable sort by (tile, depth bits), per-tile ranges.
+/* Per-tile lists of Gaussian ids in depth order, and their ranges.
  * Replaces WriteTileRecordsKernel, DeviceRadixSort::SortPairs and IdentifyTileOffsetsKernel
  * (renderer.cu:223-271, 534-569). Output order equals a stable sort of the reference keys
  * (tile << 32 | float_bits(depth)) over records enumerated in Gaussian-id order.
