@@ -5,16 +5,17 @@
 //   2. 30-bit Morton code of each point over the box (10 bits per axis), stable radix sort,
 //   3. points gathered into Morton order; axis-aligned boxes of each 8 consecutive points (the
 //      leaves) and of each 8 consecutive boxes of the level below,
-//   4. eight lanes search for one point: they test the eight children of a node together, go on with
-//      the nearest and leave the others, with their distances, on a stack in LDS; a leaf's eight
-//      points are tested the same way. A box is left out only when its lower bound is strictly
+//   4. eight lanes search for one point, from its own leaf upwards: they test the eight children of a
+//      node together, go on with the nearest and leave the others, with their distances, on a stack
+//      in LDS; a leaf's eight points are tested the same way. When nothing waits, the next ancestor's
+//      other children follow. A box is left out only when its lower bound is strictly
 //      greater than the current third-best distance.
 // What bounds it: the latency of the walk's dependent loads, hidden by eight searches per wave and
 // the waves of a SIMD. One thread per point with a stack of its own took the same walk with a
 // different node in every lane and its stack in scratch memory; a wave walking for 64 points at once
 // tested nearly every block, since the sparsest of its points set the reach of all. 200,000 points
-// of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 317 (so); about 40
-// nodes and leaves a point. Letting the searches of a wave wait for each other at their leaves took
+// of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 317 (eight lanes,
+// from the root down: about 40 nodes and leaves a point), 237 (so). Letting the searches of a wave wait for each other at their leaves took
 // 389. The bounds of the points, reduced by one thread per workgroup 32 us, by all 5.
 // Candidates are ordered by (squared distance, original index), so the three neighbours are
 // unique even with duplicate points and equal the exhaustive search with the same tie rule.
@@ -28,7 +29,8 @@ namespace gsn {
 namespace {
 
 // Children of a node (a leaf's are points), and the children of its children.
-constexpr int kFan = 8;
+constexpr int kFanBits = 3;
+constexpr int kFan = 1 << kFanBits;
 constexpr int kFan2 = kFan * kFan;
 // Levels of boxes of 2^31 points (level 0 = leaves), the root's children being the last of at most
 // kFan boxes.
@@ -256,7 +258,7 @@ constexpr int kNodeBits = 28;
 // The root's children and then seven a level can wait at once.
 constexpr int kStack = kFan * kMaxLevels;
 // Waves of a workgroup, which ends with its longest search: 328 us with four, 317 with two, 318 with
-// one (200,000 points).
+// one (200,000 points, from the root down).
 constexpr int kQueryWaves = 2;
 
 // The value of another lane of the aligned eight: across pairs, across halves of four (mirrored) or
@@ -310,7 +312,8 @@ __global__ __launch_bounds__(64 * kQueryWaves) void knn_query_kernel(const float
     const int own_leaf = static_cast<int>(k / kFan);
     int size = 0;
     uint32_t node = static_cast<uint32_t>(own_leaf);  // level 0: the leaf
-    bool own = true;
+    // Upwards from the point's own leaf: when nothing waits, the next ancestor's other children.
+    int ancestor = 1;
 #pragma unroll 1
     while (true) {
         const int level = static_cast<int>(node >> kNodeBits);
@@ -322,7 +325,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void knn_query_kernel(const float
             const float4 other = sorted[index];
             const float d = point_distance(p, other);
             const int id = __float_as_int(other.w);
-            bool open = d <= best.d2 && id != self && (own || number != own_leaf);  // false for NaN
+            bool open = d <= best.d2 && id != self;  // false for NaN
             // The nearest (the smallest id of equals) of the points that can enter the list, until
             // none is left: three at most.
             while (true) {
@@ -334,15 +337,11 @@ __global__ __launch_bounds__(64 * kQueryWaves) void knn_query_kernel(const float
                 consider(best, near, near_id);
                 open = open && id != near_id;
             }
-            if (own) {
-                own = false;
-                node = static_cast<uint32_t>(levels.top + 1) << kNodeBits;  // the root
-                next = true;
-            }
         }
         else {
             const uint32_t below = static_cast<uint32_t>(level - 1) << kNodeBits;
-            bool needed = index < s_counts[level - 1];
+            // An ancestor's child on the way to the own leaf has been walked.
+            bool needed = index < s_counts[level - 1] && index != own_leaf >> (kFanBits * (level - 1));
             float d = inf;
             if (needed) {
                 d = box_distance(p, boxes[s_offsets[level - 1] + index]);
@@ -371,7 +370,11 @@ __global__ __launch_bounds__(64 * kQueryWaves) void knn_query_kernel(const float
             next = top.distance <= best.d2;
         }
         if (!next) {
-            break;
+            if (ancestor > levels.top + 1) {
+                break;
+            }
+            node = static_cast<uint32_t>(ancestor) << kNodeBits | static_cast<uint32_t>(own_leaf >> (kFanBits * ancestor));
+            ++ancestor;
         }
     }
     if (child != 0) {
