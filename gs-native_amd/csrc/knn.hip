@@ -8,15 +8,16 @@
 //   4. eight lanes search for one point, from its own leaf upwards: they test the eight children of a
 //      node together, go on with the nearest and leave the others, with their distances, on a stack
 //      in LDS; a leaf's eight points are tested the same way. When nothing waits, the next ancestor's
-//      other children follow. A box is left out only when its lower bound is strictly
-//      greater than the current third-best distance.
+//      other children follow. A box is left out only when its lower bound is strictly greater than
+//      the current third-best distance.
 // What bounds it: the latency of the walk's dependent loads, hidden by eight searches per wave and
 // the waves of a SIMD. One thread per point with a stack of its own took the same walk with a
 // different node in every lane and its stack in scratch memory; a wave walking for 64 points at once
 // tested nearly every block, since the sparsest of its points set the reach of all. 200,000 points
 // of 64 blobs: the search 1,473 us (thread per point), 917 (wave per 64 points), 317 (eight lanes,
-// from the root down: about 40 nodes and leaves a point), 237 (so). Letting the searches of a wave wait for each other at their leaves took
-// 389. The bounds of the points, reduced by one thread per workgroup 32 us, by all 5.
+// from the root down: about 40 nodes and leaves a point), 237 (so). Letting the searches of a wave
+// wait for each other at their leaves was slower (389 against 318, from the root down). The bounds
+// of the points, reduced by one thread per workgroup 32 us, by all 5.
 // Candidates are ordered by (squared distance, original index), so the three neighbours are
 // unique even with duplicate points and equal the exhaustive search with the same tie rule.
 // Squared distances are (dx*dx + dy*dy) + dz*dz with FP contraction off, as in the host
