@@ -199,8 +199,9 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
     uint8_t* __restrict__ record_flags, uint8_t epoch, int record_count) {
     constexpr int kWaves = 4 / Bands;
     // A wave's records of the batch, in order: centre x, y, conic a, b | conic c, opacity, red, green |
-    // blue, 1 - opacity, band mask, lane (the last two as int bits). Every lane reads the same entry (no lane reads). Once walked, an
-    // entry's place takes the record's sums (kPartialFloats is its size too).
+    // blue, 1 - opacity, band mask, lane (the last two as int bits). Every lane reads the same entry
+    // (no lane reads). Once walked, an entry's place takes the record's sums (kPartialFloats is its
+    // size too).
     static_assert(kPartialFloats == 12, "an entry's place holds a record's sums");
     __shared__ float4 s_list[kWaves][65][3];
     __shared__ uint64_t s_hits[kWaves];
@@ -600,8 +601,9 @@ int launch_splat_backward(gsn_context* context, const Camera& cam, int count, co
     if (!splats || !order || !groups_order || !record_flags) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
-    // The epoch runs 1..127 (the flag's eighth bit says that the record has a partial). After a wrap, or in a newly allocated buffer, every byte is cleared
-    // first, so that a stale byte never equals the current epoch.
+    // The epoch runs 1..127 (the flag's eighth bit says that the record has a partial). After a wrap,
+    // or in a newly allocated buffer, every byte is cleared first, so that a stale byte never equals
+    // the current epoch.
     uint8_t next = static_cast<uint8_t>(context->record_epoch + 1);
     const size_t flag_bytes = context->slot_bytes[kSlotRecordFlags];
     if (next == kFlagPartial || context->record_flags_cleared != record_flags ||

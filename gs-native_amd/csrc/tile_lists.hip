@@ -383,10 +383,10 @@ __global__ __launch_bounds__(1024) void tile_offsets_kernel(const int* __restric
 // walk of the list and a quarter the gathering (3M Gaussians at 1920x1080: 195, 85 and 92 us of 385 with
 // four-byte corners in the list and the compiler's selects, 342 in all so; without the stores
 // themselves 371); and a workgroup's busiest region, since splats of one depth crowd together. Eight
-// waves a SIMD need at most 96 scalar registers: two workgroups then fit on a CU. Dealing out the rows of the regions evenly, with a list per region, took more
-// instructions and more time (732 against 501 us, 3M Gaussians at 1920x1080, both before the stores
-// were written out); counters in LDS and a scattered store per record 826 us; ids staged per tile in
-// LDS 1,032 us (three waves on a SIMD).
+// waves a SIMD need at most 96 scalar registers: two workgroups then fit on a CU. Dealing out the rows
+// of the regions evenly, with a list per region, took more instructions and more time (732 against
+// 501 us, 3M Gaussians at 1920x1080, both before the stores were written out); counters in LDS and a
+// scattered store per record 826 us; ids staged per tile in LDS 1,032 us (three waves on a SIMD).
 constexpr int kListEntries = 4096;
 constexpr int kRegionSide = 8;
 constexpr int kRegions = kPartTiles / 64;  // waves of a workgroup
@@ -599,7 +599,8 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
             store_row<5>(low, high, id, rows, column, row_low, row_high);
             store_row<6>(low, high, id, rows, column, row_low, row_high);
             store_row<7>(low, high, id, rows, column, row_low, row_high);
-            place += __popc(static_cast<uint32_t>(row_low & column_low)) + __popc(static_cast<uint32_t>(row_high & column_high));
+            place += __popc(static_cast<uint32_t>(row_low & column_low)) +
+                     __popc(static_cast<uint32_t>(row_high & column_high));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             queue[lane] = rest;
             queued = max(queued - 64, 0);
