@@ -217,16 +217,17 @@ __device__ __forceinline__ bool clip_to_part(uint2 rect, const PartTask& task, u
     return x0 < kPartSide && x1 > 0 && y0 < kPartSide && y1 > 0;
 }
 
-// Step 3. An entry costs about twelve instructions for the test and, where it meets the part, four
-// LDS adds, whatever its size; integer sums, so their order does not matter.
-__global__ __launch_bounds__(kPartThreads) void tile_count_kernel(const uint2* __restrict__ rects, int count,
-    ScreenGrid grid, int* __restrict__ counts) {
-    constexpr int kStride = kPartSide + 1;
-    __shared__ int s_corner[kStride * kStride];
+constexpr int kCornerStride = kPartSide + 1;
+
+// The number of the task's entries on the thread's tile of the part, by a whole workgroup of
+// kPartThreads. An entry costs about twelve instructions for the test and, where it meets the part,
+// four LDS adds, whatever its size; integer sums, so their order does not matter.
+__device__ __forceinline__ int count_entries(const uint2* __restrict__ rects, const PartTask& task,
+    int (&s_corner)[kCornerStride * kCornerStride]) {
+    constexpr int kStride = kCornerStride;
     for (int i = threadIdx.x; i < kStride * kStride; i += kPartThreads) {
         s_corner[i] = 0;
     }
-    const PartTask task = part_task(grid, static_cast<int>(blockIdx.x), count);
     __syncthreads();
     uint2 next = make_uint2(0u, 0u);
     if (task.begin + threadIdx.x < task.end) {
@@ -265,8 +266,15 @@ __global__ __launch_bounds__(kPartThreads) void tile_count_kernel(const uint2* _
     }
     __syncthreads();
     static_assert(kPartThreads == kPartTiles, "one tile per thread");
-    counts[static_cast<int64_t>(blockIdx.x) * kPartTiles + threadIdx.x] =
-        s_corner[(threadIdx.x / kPartSide) * kStride + threadIdx.x % kPartSide];
+    return s_corner[(threadIdx.x / kPartSide) * kStride + threadIdx.x % kPartSide];
+}
+
+// Step 3.
+__global__ __launch_bounds__(kPartThreads) void tile_count_kernel(const uint2* __restrict__ rects, int count,
+    ScreenGrid grid, int* __restrict__ counts) {
+    __shared__ int s_corner[kCornerStride * kCornerStride];
+    const PartTask task = part_task(grid, static_cast<int>(blockIdx.x), count);
+    counts[static_cast<int64_t>(blockIdx.x) * kPartTiles + threadIdx.x] = count_entries(rects, task, s_corner);
 }
 
 // Step 4, first half: exclusive prefixes of a part's counts over the chunks, in place, and the tiles'
@@ -308,60 +316,70 @@ __global__ __launch_bounds__(512) void tile_prefix_kernel(int* __restrict__ coun
     }
 }
 
+// a + b, 0xffffffff where that is more: sums past 32 bits still compare as more than any record count.
+__device__ __forceinline__ uint32_t add_capped(uint32_t a, uint32_t b) {
+    return __builtin_elementwise_add_sat(a, b);
+}
+
+// Inclusive sums over the lanes of a wave.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t value) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+        const uint32_t other = __shfl_up(value, offset);
+        value = add_capped(value, lane >= offset ? other : 0u);
+    }
+    return value;
+}
+
 // Step 4, second half: offsets[0 .. tiles], the exclusive prefix of the tiles' totals, by one
 // workgroup. Bound by latency: eight tiles a thread, the next 8,192 loaded meanwhile, and the results
-// go through LDS so that consecutive threads store consecutive entries.
-__global__ __launch_bounds__(1024) void tile_offsets_kernel(const int* __restrict__ totals, int tiles,
-    int64_t* __restrict__ offsets) {
-    constexpr int kItems = 8;
-    constexpr int kRound = 1024 * kItems;
-    __shared__ __align__(16) int s_out[kRound];
-    __shared__ int s_wave[16];
+// go through LDS so that consecutive threads store consecutive entries. Returns the sum.
+constexpr int kOffsetItems = 8;
+constexpr int kOffsetRound = 1024 * kOffsetItems;
+
+__device__ __forceinline__ uint32_t scan_totals(const int* totals, int tiles, int64_t* offsets,
+    uint32_t (&s_out)[kOffsetRound], uint32_t (&s_wave)[16]) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    auto load = [&](int64_t first, int (&values)[kItems]) {
+    auto load = [&](int64_t first, uint32_t (&values)[kOffsetItems]) {
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
+        for (int i = 0; i < kOffsetItems; ++i) {
             values[i] = first + i < tiles ? totals[first + i] : 0;
         }
     };
-    int carry = 0;
-    int next[kItems];
-    load(threadIdx.x * kItems, next);
-    for (int64_t base = 0; base < tiles; base += kRound) {
-        int values[kItems];
-        int sum = 0;
+    uint32_t carry = 0;
+    uint32_t next[kOffsetItems];
+    load(threadIdx.x * kOffsetItems, next);
+    for (int64_t base = 0; base < tiles; base += kOffsetRound) {
+        uint32_t values[kOffsetItems];
+        uint32_t sum = 0;
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
+        for (int i = 0; i < kOffsetItems; ++i) {
             values[i] = next[i];
-            sum += values[i];
+            sum = add_capped(sum, values[i]);
         }
-        load(base + kRound + threadIdx.x * kItems, next);
-        int inclusive = sum;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const int other = __shfl_up(inclusive, offset);
-            inclusive += lane >= offset ? other : 0;
-        }
+        load(base + kOffsetRound + threadIdx.x * kOffsetItems, next);
+        const uint32_t inclusive = wave_prefix(sum);
         if (lane == 63) {
             s_wave[wave] = inclusive;
         }
         __syncthreads();  // also ends the reads of the previous round's results
-        int running = carry + inclusive - sum;
+        uint32_t running = carry + inclusive - sum;
 #pragma unroll
         for (int w = 0; w < 16; ++w) {
-            const int total = s_wave[w];
+            const uint32_t total = s_wave[w];
             running += w < wave ? total : 0;
-            carry += total;
+            carry = add_capped(carry, total);
         }
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            s_out[threadIdx.x * kItems + i] = running;
+        for (int i = 0; i < kOffsetItems; ++i) {
+            s_out[threadIdx.x * kOffsetItems + i] = running;
             running += values[i];
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {
+        for (int i = 0; i < kOffsetItems; ++i) {
             const int64_t tile = base + i * 1024 + threadIdx.x;
             if (tile < tiles) {
                 offsets[tile] = s_out[i * 1024 + threadIdx.x];
@@ -370,6 +388,82 @@ __global__ __launch_bounds__(1024) void tile_offsets_kernel(const int* __restric
     }
     if (threadIdx.x == 0) {
         offsets[tiles] = carry;
+    }
+    return carry;
+}
+
+// The tiles' totals when the rectangles hold more than record_count records (a buffer of fixed
+// capacity, or rectangles of another projection): the lists keep the first record_count of them,
+// entry by entry, the last one's row by row. The prefixes of the chunk where that ends stay valid;
+// what its entries before the end add is counted again. By one workgroup, since no caller whose
+// arguments agree gets here.
+__device__ __forceinline__ void cut_totals(int* totals, const int* __restrict__ prefixes,
+    const uint2* __restrict__ rects, int count, const ScreenGrid& grid, uint32_t record_count,
+    int (&s_corner)[kCornerStride * kCornerStride], uint32_t (&s_wave)[16], int& s_last, uint32_t& s_kept) {
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    uint32_t before = 0;  // records of the entries before this round
+    for (int64_t base = 0; base < count && before <= record_count; base += 1024) {
+        const int64_t k = base + threadIdx.x;
+        const uint2 rect = k < count ? rects[k] : make_uint2(0u, 0u);
+        const uint32_t inclusive = wave_prefix(((rect.x >> 16) - (rect.x & 0xffff)) * ((rect.y >> 16) - (rect.y & 0xffff)));
+        uint32_t from = __shfl_up(inclusive, 1);
+        from = lane == 0 ? 0u : from;
+        if (lane == 63) {
+            s_wave[wave] = inclusive;
+        }
+        __syncthreads();
+        uint32_t waves_before = before;
+        for (int w = 0; w < 16; ++w) {
+            waves_before = add_capped(waves_before, w < wave ? s_wave[w] : 0u);
+            before = add_capped(before, s_wave[w]);
+        }
+        from = add_capped(from, waves_before);
+        if (from <= record_count && add_capped(inclusive, waves_before) > record_count) {
+            s_last = static_cast<int>(k);
+            s_kept = record_count - from;
+        }
+        __syncthreads();
+    }
+    const int last = s_last;
+    const uint2 rect = rects[last];
+    const int x0 = rect.x & 0xffff, x1 = rect.x >> 16, y0 = rect.y & 0xffff, y1 = rect.y >> 16;
+    const int first_task = last / grid.chunk * grid.parts;
+    for (int part = 0; part < grid.parts; ++part) {
+        PartTask task = part_task(grid, first_task + part, count);
+        task.end = last;
+        int total = count_entries(rects, task, s_corner);
+        total += prefixes[static_cast<int64_t>(first_task + part) * kPartTiles + threadIdx.x];
+        const int x = task.tile_x + static_cast<int>(threadIdx.x) % kPartSide;
+        const int y = task.tile_y + static_cast<int>(threadIdx.x) / kPartSide;
+        if (x < grid.tiles_x && y < grid.tiles_y) {
+            const bool kept = x >= x0 && x < x1 && y >= y0 && y < y1 &&
+                              static_cast<uint32_t>(y - y0) * static_cast<uint32_t>(x1 - x0) + (x - x0) < s_kept;
+            totals[y * grid.tiles_x + x] = total + kept;
+        }
+        __syncthreads();
+    }
+}
+
+// totals[tiles] tells the writing kernel whether the lists were cut.
+__global__ __launch_bounds__(1024) void tile_offsets_kernel(int* totals, const int* __restrict__ prefixes,
+    const uint2* __restrict__ rects, int count, ScreenGrid grid, int record_count, int64_t* offsets) {
+    static_assert(kPartThreads == 1024, "counts with the same workgroup");
+    __shared__ uint32_t s_out[kOffsetRound];
+    __shared__ int s_corner[kCornerStride * kCornerStride];
+    __shared__ uint32_t s_wave[16];
+    __shared__ int s_last;
+    __shared__ uint32_t s_kept;
+    const int tiles = grid.tiles_x * grid.tiles_y;
+    const bool cut = scan_totals(totals, tiles, offsets, s_out, s_wave) > static_cast<uint32_t>(record_count);
+    if (cut) {
+        __syncthreads();
+        cut_totals(totals, prefixes, rects, count, grid, static_cast<uint32_t>(record_count), s_corner, s_wave, s_last,
+            s_kept);
+        scan_totals(totals, tiles, offsets, s_out, s_wave);
+    }
+    if (threadIdx.x == 0) {
+        totals[tiles] = cut;
     }
 }
 
@@ -471,7 +565,7 @@ __device__ __forceinline__ void store_row(int low, int high, int id, uint32_t ro
 
 __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint2* __restrict__ rects,
     const uint32_t* __restrict__ list_ids, int count, ScreenGrid grid, const int* __restrict__ prefixes,
-    const int64_t* __restrict__ offsets, int record_count, int* __restrict__ ids) {
+    const int64_t* __restrict__ offsets, const int* __restrict__ cut_flag, int* __restrict__ ids) {
     __shared__ uint32_t s_id[kListEntries];
     __shared__ uint2 s_bits[kListEntries];  // columns and rows of the part, a bit each
     __shared__ uint2 s_queue[kRegions][128];  // id, columns | rows << 8 in the region
@@ -482,18 +576,18 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
     const PartTask task = part_task(grid, number, count);
     const int region_x = wave % (kPartSide / kRegionSide) * kRegionSide;
     const int region_y = wave / (kPartSide / kRegionSide) * kRegionSide;
-    int place = 0;  // of the lane's tile
-    bool fits = true;
+    int place = 0, end = 0;  // of the lane's tile: the next id's place, and the list's end
     {
         const int x = region_x + lane % kRegionSide, y = region_y + lane / kRegionSide;
         if (task.tile_x + x < grid.tiles_x && task.tile_y + y < grid.tiles_y) {
             const int64_t* begin = offsets + static_cast<int64_t>(task.tile_y + y) * grid.tiles_x + task.tile_x + x;
-            place = static_cast<int>(begin[0]) + prefixes[static_cast<int64_t>(number) * kPartTiles + y * kPartSide + x];
-            fits = begin[1] <= record_count;
+            end = static_cast<int>(begin[1]);
+            place = static_cast<int>(min(
+                begin[0] + prefixes[static_cast<int64_t>(number) * kPartTiles + y * kPartSide + x], begin[1]));
         }
     }
-    // A region with lists past the caller's record count (rectangles of another camera) is not written.
-    const bool writes = lanes_where(!fits) == 0;
+    // Lists that end before their last entry: every store looks at the end.
+    const bool cut = *cut_flag != 0;
     uint2* queue = s_queue[wave];
     int queued = 0;
     for (int64_t batch = task.begin; batch < task.end; batch += kListEntries) {
@@ -573,11 +667,21 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
             if (queued < 64 && (!last || queued == 0)) {
                 break;
             }
-            if (!writes) {
-                queued = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (cut) {
+#pragma unroll 1
+                for (int q = 0; q < min(queued, 64); ++q) {
+                    const uint2 entry = queue[q];
+                    if ((entry.y >> (lane % kRegionSide) & entry.y >> (kRegionSide + lane / kRegionSide) & 1) && place < end) {
+                        ids[place++] = static_cast<int>(entry.x);
+                    }
+                }
+                const uint2 rest = queue[64 + lane];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                queue[lane] = rest;
+                queued = max(queued - 64, 0);
                 continue;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             const uint2 entry = lane < queued ? queue[lane] : make_uint2(0u, 0u);
             const uint2 rest = queue[64 + lane];
             const int id = static_cast<int>(entry.x);
@@ -609,11 +713,15 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
 }
 
 // The reference's sort keys of the finished lists (optional output): a record's tile is the last one
-// that begins at or before it.
+// that begins at or before it. All ones past the last list's end, where no id was written.
 __global__ __launch_bounds__(256) void sorted_keys_kernel(const int64_t* __restrict__ offsets, int tiles,
     const int* __restrict__ ids, const float* __restrict__ depths, uint64_t* __restrict__ keys, int records) {
     int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= records) {
+        return;
+    }
+    if (r >= offsets[tiles]) {
+        keys[r] = ~0ull;
         return;
     }
     int low = 0, high = tiles;
@@ -670,7 +778,7 @@ static int enqueue_lists(gsn_context* context, const ScreenGrid& grid, int count
     const uint32_t* sorted_keys = static_cast<uint32_t*>(scratch(context, kSlotDepthSortedKeys, n * 4));
     uint2* rects = static_cast<uint2*>(scratch(context, kSlotDepthRects, n * sizeof(uint2)));
     int* counts = static_cast<int*>(scratch(context, kSlotTileCounts, static_cast<size_t>(tasks) * kPartTiles * 4));
-    int* totals = static_cast<int*>(scratch(context, kSlotTileTotals, tile_count * 4));
+    int* totals = static_cast<int*>(scratch(context, kSlotTileTotals, (tile_count + 1) * 4));
     if (!sorted_ids || !sorted_keys || !rects || !counts || !totals) {
         return GSN_ERROR_OUT_OF_MEMORY;
     }
@@ -687,12 +795,12 @@ static int enqueue_lists(gsn_context* context, const ScreenGrid& grid, int count
         GSN_TRY(check_launch("tile_count_kernel"));
         tile_prefix_kernel<<<static_cast<unsigned>(grid.parts * (kPartTiles / 64)), 512, 0, stream>>>(counts, grid, totals);
         GSN_TRY(check_launch("tile_prefix_kernel"));
-        tile_offsets_kernel<<<1, 1024, 0, stream>>>(totals, static_cast<int>(tile_count), offsets);
+        tile_offsets_kernel<<<1, 1024, 0, stream>>>(totals, counts, rects, count, grid, record_count, offsets);
         GSN_TRY(check_launch("tile_offsets_kernel"));
     }
     StageScope scope(context, kStageTileSort);
     tile_write_kernel<<<static_cast<unsigned>(tasks), 64 * kRegions, 0, stream>>>(rects, sorted_ids, count, grid,
-        counts, offsets, record_count, ids);
+        counts, offsets, totals + tile_count, ids);
     return check_launch("tile_write_kernel");
 }
 

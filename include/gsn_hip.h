@@ -170,7 +170,11 @@ int gsn_scan_record_offsets(gsn_context* context, int* record_offsets, int count
  * (renderer.cu:223-271, 534-569). Output order equals a stable sort of the reference keys
  * (tile << 32 | float_bits(depth)) over records enumerated in Gaussian-id order.
  * sorted_keys[R] is optional (NULL to skip). Reuses the depth order queued by
- * gsn_scan_record_offsets for the same depths / record_offsets / count, else computes it. */
+ * gsn_scan_record_offsets for the same depths / record_offsets / count, else computes it.
+ * Rectangles are clamped to the camera's grid. record_count is the capacity of tile_gaussian_ids
+ * and sorted_keys: when the rectangles hold more records, the lists hold the first record_count of
+ * them (nearest first, row by row inside a rectangle); when they hold fewer, the lists end before
+ * it (tile_offsets[T]), the ids from there on are unspecified and the keys all ones. */
 int gsn_build_tile_lists(gsn_context* context, const gsn_camera* camera, int count,
     const int* tile_rects, const float* depths, const int* record_offsets, int record_count,
     int* tile_gaussian_ids, int64_t* tile_offsets, uint64_t* sorted_keys);
