@@ -198,6 +198,7 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
     const float* __restrict__ image_gradients, float bg_r, float bg_g, float bg_b, float* __restrict__ partials,
     uint8_t* __restrict__ record_flags, uint8_t epoch, int record_count) {
     constexpr int kWaves = 4 / Bands;
+    constexpr bool kIfs = Stored && Bands > 1, kSelects = Stored && Bands == 1;
     // A wave's records of the batch, in order: centre x, y, conic a, b | conic c, opacity, red, green |
     // blue, 1 - opacity, band mask, lane (the last two as int bits). Every lane reads the same entry
     // (no lane reads). Once walked, an entry's place takes the record's sums (kPartialFloats is its
@@ -316,10 +317,12 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
         const uint64_t hits = lanes_where(mask != 0);
         if (mask != 0) {
             const int place = lanes_below(hits);
+            // No pixel is below the cap with an opacity that is not finite: its factor is not needed.
+            const float rest = Stored && !isfinite(conic.w) ? 0.0f : 1.0f - conic.w;
             s_list[wave][place][0] = make_float4(following.a.x, following.a.y, conic.x, conic.y);
             s_list[wave][place][1] = make_float4(conic.z, conic.w, following.b.z, following.b.w);
             s_list[wave][place][2] =
-                make_float4(following.c.x, 1.0f - conic.w, __int_as_float(mask), __int_as_float(lane));
+                make_float4(following.c.x, rest, __int_as_float(mask), __int_as_float(lane));
         }
         if (wave == 0) {
             s_slot[lane] = valid ? static_cast<int>(partial_slot(following.c, tile_x, tile_y)) : -1;
@@ -373,39 +376,49 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
                     const uint64_t open = Stored ? lanes_where(tile_index + __float_as_int(c4.w) < p.last)
                                                  : lanes_where(next >= kTransmittanceMin);
                     const uint64_t blend = take & open;
-                    // Uniform branch on "some lane blends"; inside, lanes that do not blend add
-                    // exact zeros (selects, not divergent ifs), which keeps the accumulators in
-                    // place instead of merging per-lane control paths.
+                    // Uniform branch on "some lane blends". Recompute form: inside, lanes that do not
+                    // blend add exact zeros (selects, not divergent ifs), which keeps the accumulators
+                    // in place instead of merging per-lane control paths. Stored form: lanes that do
+                    // not blend stay out, so that a gradient, colour or conic that is not finite
+                    // reaches only the sums of splats blended at its pixel (0 times it would not be 0):
+                    // by divergent ifs with four bands a wave (4,108 tiles of 400 records: 398 us, without
+                    // them 399, selects 435), by selects with one, where ifs need the sums' zeros in
+                    // registers first (1,024 tiles of 300: 130 us, without them 127, ifs 138).
                     if (blend) {
                         blended |= blend;
                         const float inv = __builtin_amdgcn_rcpf(through);
                         const float before = Stored ? p.T * inv : p.T;
-                        const float weight = in_lanes(blend) ? alpha * before : 0.0f;
+                        const float weight = kIfs || in_lanes(blend) ? alpha * before : 0.0f;
                         const float colour[3] = {b4.z, b4.w, c4.x};
-                        float sum = 0.0f;
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            const float difference = Stored ? fmaf(before, colour[c], -p.walked[c] * inv)
-                                                            : fmaf(colour[c], before, p.walked[c]) - p.final[c];
-                            sum = Stored ? fmaf(p.grad[c], difference, sum) : fmaf(inv, p.grad[c] * difference, sum);
-                            acc[6 + c] = fmaf(weight, p.grad[c], acc[6 + c]);
-                            p.walked[c] = fmaf(colour[c], weight, p.walked[c]);
-                        }
                         const uint64_t uncapped = blend & lanes_where(raw_alpha < kAlphaMax);
-                        const float common = in_lanes(uncapped) ? raw_alpha * sum : 0.0f;
-                        const float qx = fmaf(cbv, dy, ca_dx);
-                        const float qy = along + cc * dy;
-                        const float gx = common * qx;
-                        const float gy = common * qy;
-                        acc[0] = fmaf(qx, common, acc[0]);
-                        acc[1] = fmaf(qy, common, acc[1]);
-                        acc[2] = fmaf(qx, gx, acc[2]);
-                        acc[3] = fmaf(qy, gx, acc[3]);
-                        acc[4] = fmaf(qy, gy, acc[4]);
-                        acc[5] = fmaf(c4.y, common, acc[5]);
-                        acc[9] += fabsf(gx);
-                        acc[10] += fabsf(gy);
-                        p.T = in_lanes(blend) ? (Stored ? before : next) : p.T;
+                        if (!kIfs || in_lanes(blend)) {
+                            float sum = 0.0f;
+#pragma unroll
+                            for (int c = 0; c < 3; ++c) {
+                                const float difference = Stored ? fmaf(before, colour[c], -p.walked[c] * inv)
+                                                                : fmaf(colour[c], before, p.walked[c]) - p.final[c];
+                                sum = Stored ? fmaf(p.grad[c], difference, sum) : fmaf(inv, p.grad[c] * difference, sum);
+                                acc[6 + c] = fmaf(weight, !kSelects || in_lanes(blend) ? p.grad[c] : 0.0f, acc[6 + c]);
+                                const float walked = fmaf(colour[c], weight, p.walked[c]);
+                                p.walked[c] = !kSelects || in_lanes(blend) ? walked : p.walked[c];
+                            }
+                            p.T = in_lanes(blend) ? (Stored ? before : next) : p.T;
+                            if (!kIfs || in_lanes(uncapped)) {
+                                const float common = in_lanes(uncapped) ? raw_alpha * sum : 0.0f;
+                                const float qx = !kSelects || in_lanes(uncapped) ? fmaf(cbv, dy, ca_dx) : 0.0f;
+                                const float qy = !kSelects || in_lanes(uncapped) ? along + cc * dy : 0.0f;
+                                const float gx = common * qx;
+                                const float gy = common * qy;
+                                acc[0] = fmaf(qx, common, acc[0]);
+                                acc[1] = fmaf(qy, common, acc[1]);
+                                acc[2] = fmaf(qx, gx, acc[2]);
+                                acc[3] = fmaf(qy, gx, acc[3]);
+                                acc[4] = fmaf(qy, gy, acc[4]);
+                                acc[5] = fmaf(c4.y, common, acc[5]);
+                                acc[9] += fabsf(gx);
+                                acc[10] += fabsf(gy);
+                            }
+                        }
                     }
                     if (!Stored && (take & ~open)) {
                         keep(p.T);
