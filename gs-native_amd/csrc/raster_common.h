@@ -85,7 +85,7 @@ __device__ __forceinline__ float splat_alpha(float across, float along, float c,
 // Per band, the region's x-range is taken over the band's rows only (the slab's extremes of the
 // ellipse's chords; the ellipse's own extreme point when it lies inside the slab), with the same
 // 2% + 0.5 px margin and never wider than the whole-tile test: a band is kept only if that range
-// meets the tile's 16 columns. Non-finite inputs keep every band. The hardware's one-ulp reciprocal,
+// meets the tile's 16 columns. Non-finite and extreme inputs keep every band. The hardware's one-ulp reciprocal,
 // square root and logarithm are far inside the margins (the correctly rounded forms made the mask
 // several times longer).
 // Tests the `Bands` bands from first_band on; bit b stands for band first_band + b.
@@ -97,7 +97,11 @@ __device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x
         return (o == o) ? 0 : kAll;
     }
     float det = a * c - b * b;
-    if (!(det > 0.0f) || !isfinite(det) || !isfinite(mx) || !isfinite(my)) {
+    // det, a and c inside the range where their reciprocals and they themselves are normal numbers: the
+    // hardware's reciprocal takes a subnormal operand for zero and gives zero for a subnormal result.
+    constexpr float kSmallest = 0x1p-125f, kLargest = 0x1p125f;
+    if (!(det >= kSmallest) || !(fminf(a, c) >= kSmallest) || !(fmaxf(det, fmaxf(a, c)) <= kLargest) ||
+        !isfinite(mx) || !isfinite(my)) {
         return kAll;
     }
     float tau = __logf(255.0f * o) + 0.25f;
