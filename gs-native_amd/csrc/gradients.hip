@@ -405,7 +405,7 @@ __device__ __forceinline__ void reduce_records(const float* __restrict__ partial
             slots[3 * (64 + lane) + 1] = b1;
             slots[3 * (64 + lane) + 2] = c1;
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
             // This lane's records [begin, end) within the chunk.
@@ -473,7 +473,7 @@ __device__ __forceinline__ void reduce_records(const float* __restrict__ partial
                 in[10] += cc.z;
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
 }
 

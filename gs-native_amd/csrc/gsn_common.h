@@ -266,4 +266,11 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
     return base + idx;
 }
 
+// Between LDS accesses of one wave: what its lanes wrote before, any of them reads after. The hardware
+// runs a wave's LDS instructions in order; this keeps the compiler from moving or merging them.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 } // namespace gsn

@@ -364,6 +364,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void knn_query_kernel(const float
                 next = true;
             }
         }
+        wave_lds_fence();
         // Else the next box that can still hold a candidate.
         while (!next && size > 0) {
             const Waiting top = stack[--size];

@@ -332,13 +332,13 @@ __global__ __launch_bounds__(64 * kMlpWaves, 1) void mlp_gradient_kernel(const f
                 gb3[c] += static_cast<float>(dz3[c]);
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         bf16x8 dz3t[2];
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             dz3t[c] = n < kClasses ? *reinterpret_cast<const bf16x8*>(&s_dz3[wave][n][16 * c + k8]) : zero_operand();
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         // By feature: the activations of both layers, and dZ2 and dZ1 with them.
         bf16x8 dz2[4], dz2t[2][2], a1t[2][2];
         float z1t[2][16];

@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
             s_wave_count[wave][digit] = count + __popcll(peers);
         }
         // Keeps the next round's counter reads after this round's leader writes.
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
     __syncthreads();
 

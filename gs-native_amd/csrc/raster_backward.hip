@@ -335,7 +335,7 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
         uint64_t contributed = 0;
         const int entries = __popcll(hits);
         auto place_of = [&](int step) { return Stored ? entries - 1 - step : step; };
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         float4 next_a = s_list[wave][max(place_of(0), 0)][0];
         float4 next_b = s_list[wave][max(place_of(0), 0)][1];
         float4 next_c = s_list[wave][max(place_of(0), 0)][2];

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(64) void raster_forward_kernel(const int* __restric
             load(following_id);
         }
         following_id = base + 128 + lane < end ? ids[base + 128 + lane] : -1;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
         const int entries = __popcll(hits);
         ForwardEntry next_entry = s_list[0];
         for (int k = 0; k < entries; ++k) {
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(64) void raster_forward_kernel(const int* __restric
                 }
             });
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
     each([&](ForwardPixel& p, int b) {
         const int y = py + 4 * b;

@@ -667,7 +667,7 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
             if (queued < 64 && (!last || queued == 0)) {
                 break;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            wave_lds_fence();
             if (cut) {
 #pragma unroll 1
                 for (int q = 0; q < min(queued, 64); ++q) {
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
                     }
                 }
                 const uint2 rest = queue[64 + lane];
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                wave_lds_fence();
                 queue[lane] = rest;
                 queued = max(queued - 64, 0);
                 continue;
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(64 * kRegions, 8) void tile_write_kernel(const uint
             store_row<7>(low, high, id, rows, column, row_low, row_high);
             place += __popc(static_cast<uint32_t>(row_low & column_low)) +
                      __popc(static_cast<uint32_t>(row_high & column_high));
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            wave_lds_fence();
             queue[lane] = rest;
             queued = max(queued - 64, 0);
         }
