@@ -477,7 +477,7 @@ __global__ __launch_bounds__(1024) void tile_offsets_kernel(int* totals, const i
 // walk of the list and a quarter the gathering (3M Gaussians at 1920x1080: 195, 85 and 92 us of 385 with
 // four-byte corners in the list and the compiler's selects, 342 in all so; without the stores
 // themselves 371); and a workgroup's busiest region, since splats of one depth crowd together. Eight
-// waves a SIMD need at most 96 scalar registers: two workgroups then fit on a CU. Dealing out the rows
+// waves a SIMD let two workgroups fit on a CU. Dealing out the rows
 // of the regions evenly, with a list per region, took more instructions and more time (732 against
 // 501 us, 3M Gaussians at 1920x1080, both before the stores were written out); counters in LDS and a
 // scattered store per record 826 us; ids staged per tile in LDS 1,032 us (three waves on a SIMD).
@@ -487,12 +487,15 @@ constexpr int kRegions = kPartTiles / 64;  // waves of a workgroup
 
 // For every lane the mask of its tile's column (low, high), under one constant lane mask per column:
 // three instructions a column where a select takes six.
+// The scalar registers named here and in store_row are below the 74 that the compiler gives out at
+// eight waves a SIMD. With s76 to s81, which are reserved then (it warns that such need not be
+// preserved), the kernel also allocated more of them: 2M Gaussians at 3840x2160 1,328 us a render, 1,282 so.
 __device__ __forceinline__ void column_masks(const uint64_t (&column)[8], int& low, int& high) {
 #define GSN_COLUMN(low_half, high_half, next) \
     "v_mov_b32 %[low], " low_half "\nv_mov_b32 %[high], " high_half "\n" next
 #define GSN_NEXT_COLUMN "s_lshl_b64 exec, exec, 1\n"
     auto half = [&](int i, int part) { return static_cast<uint32_t>(column[i] >> (32 * part)); };
-    asm volatile("s_mov_b64 s[80:81], exec\n"
+    asm volatile("s_mov_b64 s[64:65], exec\n"
         "s_mov_b32 exec_lo, 0x01010101\n"
         "s_mov_b32 exec_hi, 0x01010101\n"
         GSN_COLUMN("%[l0]", "%[h0]", GSN_NEXT_COLUMN)
@@ -503,13 +506,13 @@ __device__ __forceinline__ void column_masks(const uint64_t (&column)[8], int& l
         GSN_COLUMN("%[l5]", "%[h5]", GSN_NEXT_COLUMN)
         GSN_COLUMN("%[l6]", "%[h6]", GSN_NEXT_COLUMN)
         GSN_COLUMN("%[l7]", "%[h7]", "")
-        "s_mov_b64 exec, s[80:81]"
+        "s_mov_b64 exec, s[64:65]"
         : [low] "+v"(low), [high] "+v"(high)
         : [l0] "s"(half(0, 0)), [h0] "s"(half(0, 1)), [l1] "s"(half(1, 0)), [h1] "s"(half(1, 1)),
         [l2] "s"(half(2, 0)), [h2] "s"(half(2, 1)), [l3] "s"(half(3, 0)), [h3] "s"(half(3, 1)),
         [l4] "s"(half(4, 0)), [h4] "s"(half(4, 1)), [l5] "s"(half(5, 0)), [h5] "s"(half(5, 1)),
         [l6] "s"(half(6, 0)), [h6] "s"(half(6, 1)), [l7] "s"(half(7, 0)), [h7] "s"(half(7, 1))
-        : "s80", "s81", "scc");
+        : "s64", "s65", "scc");
 #undef GSN_COLUMN
 #undef GSN_NEXT_COLUMN
 }
@@ -536,21 +539,21 @@ __device__ __forceinline__ void store_row(int low, int high, int id, uint32_t ro
     "global_store_dword %[offset], %[id], s[" now "]\n"
 #define GSN_NEXT_TILE(first, second, tile) \
     "v_readlane_b32 s" first ", %[low], " tile "\nv_readlane_b32 s" second ", %[high], " tile "\n"
-    asm volatile("s_mov_b64 s[80:81], exec\n"
+    asm volatile("s_mov_b64 s[64:65], exec\n"
         "s_mov_b32 exec_lo, %[lanes_low]\n"
         "s_mov_b32 exec_hi, %[lanes_high]\n"
         "v_mov_b32 %[row_low], %[mask_low]\n"
         "v_mov_b32 %[row_high], %[mask_high]\n"
-        GSN_NEXT_TILE("76", "77", "%[t0]")
-        GSN_STORE_TILE("%[c0]", "76:77", GSN_NEXT_TILE("78", "79", "%[t1]"))
-        GSN_STORE_TILE("%[c1]", "78:79", GSN_NEXT_TILE("76", "77", "%[t2]"))
-        GSN_STORE_TILE("%[c2]", "76:77", GSN_NEXT_TILE("78", "79", "%[t3]"))
-        GSN_STORE_TILE("%[c3]", "78:79", GSN_NEXT_TILE("76", "77", "%[t4]"))
-        GSN_STORE_TILE("%[c4]", "76:77", GSN_NEXT_TILE("78", "79", "%[t5]"))
-        GSN_STORE_TILE("%[c5]", "78:79", GSN_NEXT_TILE("76", "77", "%[t6]"))
-        GSN_STORE_TILE("%[c6]", "76:77", GSN_NEXT_TILE("78", "79", "%[t7]"))
-        GSN_STORE_TILE("%[c7]", "78:79", "")
-        "s_mov_b64 exec, s[80:81]"
+        GSN_NEXT_TILE("60", "61", "%[t0]")
+        GSN_STORE_TILE("%[c0]", "60:61", GSN_NEXT_TILE("62", "63", "%[t1]"))
+        GSN_STORE_TILE("%[c1]", "62:63", GSN_NEXT_TILE("60", "61", "%[t2]"))
+        GSN_STORE_TILE("%[c2]", "60:61", GSN_NEXT_TILE("62", "63", "%[t3]"))
+        GSN_STORE_TILE("%[c3]", "62:63", GSN_NEXT_TILE("60", "61", "%[t4]"))
+        GSN_STORE_TILE("%[c4]", "60:61", GSN_NEXT_TILE("62", "63", "%[t5]"))
+        GSN_STORE_TILE("%[c5]", "62:63", GSN_NEXT_TILE("60", "61", "%[t6]"))
+        GSN_STORE_TILE("%[c6]", "60:61", GSN_NEXT_TILE("62", "63", "%[t7]"))
+        GSN_STORE_TILE("%[c7]", "62:63", "")
+        "s_mov_b64 exec, s[64:65]"
         : [offset] "=&v"(offset), [row_low] "+&v"(row_low), [row_high] "+&v"(row_high)
         : [low] "v"(low), [high] "v"(high), [id] "v"(id), [row] "s"(row), [c0] "s"(column[0]), [c1] "s"(column[1]),
         [c2] "s"(column[2]), [c3] "s"(column[3]), [c4] "s"(column[4]), [c5] "s"(column[5]), [c6] "s"(column[6]),
@@ -558,7 +561,7 @@ __device__ __forceinline__ void store_row(int low, int high, int id, uint32_t ro
         [lanes_low] "n"(Row < 4 ? 0xff << (8 * (Row & 3)) : 0), [lanes_high] "n"(Row < 4 ? 0 : 0xff << (8 * (Row & 3))),
         [t0] "n"(8 * Row), [t1] "n"(8 * Row + 1), [t2] "n"(8 * Row + 2), [t3] "n"(8 * Row + 3),
         [t4] "n"(8 * Row + 4), [t5] "n"(8 * Row + 5), [t6] "n"(8 * Row + 6), [t7] "n"(8 * Row + 7)
-        : "s76", "s77", "s78", "s79", "s80", "s81", "scc", "memory");
+        : "s60", "s61", "s62", "s63", "s64", "s65", "scc", "memory");
 #undef GSN_STORE_TILE
 #undef GSN_NEXT_TILE
 }
