@@ -15,15 +15,18 @@ enum ScratchSlot {
     kSlotSortKeysA = 0,
     kSlotSortKeysB,
     kSlotSortValuesA,
-    kSlotSortValuesB,
     kSlotSortHistogram,
     kSlotScanBlocks,
     kSlotDepthKeys,
     kSlotDepthIds,
-    kSlotDepthOffsets,
     kSlotDepthSortedIds,
     kSlotTileCounts,
     kSlotTileTotals,
+    kSlotDepthCounts,
+    kSlotDepthCountTotals,
+    kSlotRecordTiles,
+    kSlotRecordIds,
+    kSlotEmitOwners,
     kSlotPartials,
     kSlotReduce,
     kSlotKnnKeys,
@@ -184,6 +187,13 @@ struct Int4 {
 };
 int exclusive_scan_int(gsn_context* context, const int* input, int* output, int64_t n);
 int exclusive_scan_int4(gsn_context* context, const Int4* input, Int4* output, int64_t n);
+// Exclusive scan of values that are not negative, with sums that stay at the largest int instead of
+// wrapping. The producer of `input` has written the sum of each kScanBlock-element block (entries
+// [b * kScanBlock, (b + 1) * kScanBlock) of [0, n)) to block_totals[b]: only the downsweep runs (beyond
+// 2048 blocks the totals are ignored and the full scan runs).
+constexpr int kScanBlock = 4096;
+int exclusive_scan_capped_from_totals(gsn_context* context, const int* input, int* output, int64_t n,
+    const int* block_totals);
 
 // Stable LSD radix sort of (uint32 key, uint32 value) pairs over key bits [0, bits)
 // (radix_sort.hip). Input buffers are consumed. The result is written to keys_out/values_out
@@ -203,6 +213,11 @@ int* radix_histogram_buffer(gsn_context* context, int64_t n);
 int radix_first_digit_bits(int bits);
 int radix_sort_pairs(gsn_context* context, uint32_t* keys, uint32_t* values, int64_t n,
     int bits, uint32_t* keys_out, uint32_t* values_out, bool first_histogram_ready = false);
+
+// The per-tile lists from the depth order in kSlotDepthSortedIds / Keys, by sorting the records
+// (record_lists.hip): ids[0 .. record_count) and offsets[0 .. tiles].
+int enqueue_lists_by_records(gsn_context* context, int tiles_x, int tiles_y, int count, const int4* tile_rects,
+    int record_count, int* ids, int64_t* offsets);
 
 // Floats per (tile, Gaussian) backward partial: dmean2D(2), dSigma2D(3), dlogit, dcolor(3),
 // |dmean2D|(2), pad.

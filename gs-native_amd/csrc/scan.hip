@@ -1,7 +1,7 @@
 // Device-wide exclusive prefix scan: per-block totals, then a downsweep in which every block adds
 // the totals of the blocks before it (summed directly up to 2048 blocks, else from a recursive
 // scan of the totals).
-// Used for record offsets (int[N+1]) and density decisions (int4[N+1]).
+// Used for record offsets (int[N+1]), depth-order record counts and density decisions (int4[N+1]).
 #include "gsn_internal.h"
 
 namespace gsn {
@@ -12,6 +12,12 @@ namespace {
 constexpr int kScanThreads = 512;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
+static_assert(kScanTile == kScanBlock, "block totals written by producers cover kScanBlock entries");
+
+// A sum that stays at the largest int instead of wrapping.
+struct Capped {
+    int value;
+};
 
 __device__ __forceinline__ int add(int a, int b) {
     return a + b;
@@ -21,8 +27,17 @@ __device__ __forceinline__ Int4 add(Int4 a, Int4 b) {
     return Int4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
 }
 
+__device__ __forceinline__ Capped add(Capped a, Capped b) {
+    return Capped{__builtin_elementwise_add_sat(a.value, b.value)};
+}
+
 template<typename T>
 __device__ __forceinline__ T zero_value();
+
+template<>
+__device__ __forceinline__ Capped zero_value<Capped>() {
+    return Capped{0};
+}
 
 template<>
 __device__ __forceinline__ int zero_value<int>() {
@@ -40,6 +55,10 @@ __device__ __forceinline__ int shuffle_up(int v, int d) {
 
 __device__ __forceinline__ Int4 shuffle_up(Int4 v, int d) {
     return Int4{__shfl_up(v.x, d, 64), __shfl_up(v.y, d, 64), __shfl_up(v.z, d, 64), __shfl_up(v.w, d, 64)};
+}
+
+__device__ __forceinline__ Capped shuffle_up(Capped v, int d) {
+    return Capped{__shfl_up(v.value, d, 64)};
 }
 
 // Inclusive scan across the 64 lanes of a wave.
@@ -167,6 +186,28 @@ __device__ __forceinline__ void store_items(Int4* output, int64_t base, int64_t 
     }
 }
 
+static_assert(sizeof(Capped) == sizeof(int), "loaded and stored as int");
+
+__device__ __forceinline__ void load_items(const Capped* input, int64_t base, int64_t n, bool vector,
+    Capped (&items)[kScanItems]) {
+    int values[kScanItems];
+    load_items(reinterpret_cast<const int*>(input), base, n, vector, values);
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) {
+        items[i].value = values[i];
+    }
+}
+
+__device__ __forceinline__ void store_items(Capped* output, int64_t base, int64_t n, bool vector,
+    const Capped (&items)[kScanItems]) {
+    int values[kScanItems];
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) {
+        values[i] = items[i].value;
+    }
+    store_items(reinterpret_cast<int*>(output), base, n, vector, values);
+}
+
 // Exclusive scan of each kScanTile block, offset by the sum of all earlier blocks: with
 // sum_totals the block adds up block_totals[0 .. block) itself, otherwise block_totals already
 // holds the exclusive scan of the totals and entry [block] is the offset. In-place use (input == output) is allowed: every
@@ -252,6 +293,20 @@ int exclusive_scan(gsn_context* context, const T* input, T* output, int64_t n, i
 
 int exclusive_scan_int(gsn_context* context, const int* input, int* output, int64_t n) {
     return exclusive_scan<int>(context, input, output, n, 0);
+}
+
+int exclusive_scan_capped_from_totals(gsn_context* context, const int* input, int* output, int64_t n,
+    const int* block_totals) {
+    const Capped* in = reinterpret_cast<const Capped*>(input);
+    Capped* out = reinterpret_cast<Capped*>(output);
+    const int64_t blocks = (n + kScanTile - 1) / kScanTile;
+    if (n <= 0 || blocks == 1 || blocks > kSumTotalsBlocks) {
+        return exclusive_scan<Capped>(context, in, out, n, 0);
+    }
+    const int vector = (reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(output) % 16 == 0) ? 1 : 0;
+    scan_downsweep_kernel<Capped><<<static_cast<unsigned>(blocks), kScanThreads, 0, context->stream>>>(in, out,
+        reinterpret_cast<const Capped*>(block_totals), n, 1, vector);
+    return check_launch("scan_downsweep_kernel");
 }
 
 int exclusive_scan_int4(gsn_context* context, const Int4* input, Int4* output, int64_t n) {

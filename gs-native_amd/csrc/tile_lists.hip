@@ -19,6 +19,7 @@
 // instructions. Emission to ranges with the sort and so: 10K Gaussians at 256x256 45 and 25 us, 200K
 // at 979x546 88 and 73, 500K at 1248x832 160 and 113, 3M at 1920x1080 660 and 494, 2M at 3840x2160
 // 2,100 and 640.
+// Lists with few records per entry and part are sorted after all (lists_by_records).
 #include "raster_common.h"
 
 #include <algorithm>
@@ -771,6 +772,20 @@ static ScreenGrid screen_grid(int count, int tiles_x, int tiles_y) {
     return grid;
 }
 
+// Whether sorting the records (record_lists.hip) is the shorter way: its cost goes with the records,
+// that of counting and writing with the tests of every list entry against every part, which are many
+// where most Gaussians are culled or cover a tile or two of a large screen. Of 165 lists of 0.2M to 6M
+// Gaussians at 1248x832 to 5187x3361 the sort is the shorter way below 0.2 records per test and the
+// longer one above 0.38; between, it depends on how many are visible, which is not known here. In all, by
+// records and by counting: 3M at 1920x1080, 5% visible, 0.7M records 69 and 131 us, 30% 8M 168 and 173,
+// all 27M 443 and 303; 2M at 3840x2160, 5% 0.9M 69 and 244, all 18M 323 and 406, all 30M 526 and 409; 4M at
+// 5187x3361, 5% 1.8M 104 and 798. Below 4M tests (0.3M at 1920x1080, 5%: 47 and 51 us) counting's fewer
+// launches decide.
+static bool lists_by_records(const ScreenGrid& grid, int count, int record_count) {
+    const int64_t tests = static_cast<int64_t>(count) * grid.parts;
+    return tests > 4'000'000 && 4 * static_cast<int64_t>(record_count) < tests;
+}
+
 // The lists, from the depth order: steps 2 to 5.
 static int enqueue_lists(gsn_context* context, const ScreenGrid& grid, int count, const int4* tile_rects,
     int record_count, int* ids, int64_t* offsets) {
@@ -915,7 +930,10 @@ extern "C" int gsn_build_tile_lists(gsn_context* context, const gsn_camera* came
     }
     const ScreenGrid grid = screen_grid(count, camera->tile_count_x, camera->tile_count_y);
     const int4* rects = reinterpret_cast<const int4*>(tile_rects);
-    GSN_TRY(enqueue_lists(context, grid, count, rects, record_count, tile_gaussian_ids, tile_offsets));
+    GSN_TRY(lists_by_records(grid, count, record_count)
+                ? enqueue_lists_by_records(context, grid.tiles_x, grid.tiles_y, count, rects, record_count, tile_gaussian_ids,
+                      tile_offsets)
+                : enqueue_lists(context, grid, count, rects, record_count, tile_gaussian_ids, tile_offsets));
     if (sorted_keys) {
         sorted_keys_kernel<<<grid_for(record_count, 256), 256, 0, stream>>>(tile_offsets, tile_count, tile_gaussian_ids,
             depths, sorted_keys, record_count);

@@ -85,8 +85,9 @@ int gsn_device_memory_info(size_t* free_bytes, size_t* total_bytes);
  * cv::TickMeter). While enabled, every stage records a HIP event pair on the context stream;
  * gsn_context_stage_times synchronises, returns the summed milliseconds and the number of timed
  * launches of each stage, and clears the record. Stage order:
- *   0 project, 1 scan, 2 depth sort, 3 rectangles in depth order, 4 tile lists' ids written,
- *   5 tile counts and offsets,
+ *   0 project, 1 scan, 2 depth sort, 3 rectangles in depth order (lists by records: with the
+ *   records emitted), 4 tile lists' ids written (records sorted), 5 tile counts and offsets
+ *   (ranges of the sorted records),
  *   6 raster forward, 7 image gradients, 8 raster backward, 9 per-Gaussian gradients (+Adam),
  *   10 Adam, 11 density control (count, write, history remap, opacity cap), 12 KNN,
  *   13 statistics accumulation (per-view density and feature accumulators). */

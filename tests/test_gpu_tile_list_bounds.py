@@ -96,7 +96,7 @@ def test_more_records_than_32_bits(gsn, context):
     grid, count = (512, 511), 20_000
     rects = np.tile(np.array([0, 0, *grid]), (count, 1))
     depths = np.random.default_rng(1).permutation(count).astype(np.float32) + 1
-    _check(gsn, context, grid, rects, depths, np.ones(count, bool), 700_001)
+    _check(gsn, context, grid, rects, depths, np.ones(count, bool), 1_300_001)
 
 
 def test_cut_lists_render(gsn, context, scenes):
