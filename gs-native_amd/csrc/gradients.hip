@@ -645,10 +645,15 @@ __global__ __launch_bounds__(256) void adam_kernel(const float* __restrict__ gra
 // One thread per new Gaussian: its parent id is read once and its 58 moment pairs are gathered
 // kRemapRows rows at a time (all loads of a group in flight); neighbouring new ids mostly have
 // neighbouring parents, so each row's gathers and stores stay within one or two 512-byte pieces.
-// Bound by memory; both sides are read or written once and larger than the caches: non-temporal
-// (500K Gaussians: 126 -> 111 us, the parameters' copy beside it 84 -> 79).
+// Bound by memory; both sides are read or written once. Streaming: non-temporal accesses, where both
+// sides together exceed the 256 MB of the last-level cache; below that the previous moments are still
+// there from the step before, and the new ones are wanted by the step after. Non-temporal and plain,
+// right after an Adam step: 50K Gaussians 15.0 and 13.4 us, 100K 23.2 and 18.7, 200K 43.2 and 34.6 (with
+// the next Adam step 97.6 and 96.4), 300K 57.6 and 57.6 (139 and 148), 1M 183 and 188, 3M 536 and 555.
 constexpr int kRemapRows = 8;
+constexpr int64_t kStreamedBytes = 256ll << 20;
 
+template<bool Streaming>
 __global__ __launch_bounds__(256) void remap_history_kernel(const int* parent_ids, const float* previous, float* moments,
     int previous_count, int count) {
     int id = blockIdx.x * blockDim.x + threadIdx.x;
@@ -659,20 +664,33 @@ __global__ __launch_bounds__(256) void remap_history_kernel(const int* parent_id
     const bool inherited = parent >= 0 && parent < previous_count;
 #pragma unroll
     for (int base = 0; base < kParamCount; base += kRemapRows) {
-        moment_pair pairs[kRemapRows];
+        float2 pairs[kRemapRows];  // not vectors, whose zeros and loads the compiler merges lane by lane
 #pragma unroll
         for (int k = 0; k < kRemapRows; ++k) {
             const int row = base + k;
-            pairs[k] = moment_pair{0.0f, 0.0f};
+            pairs[k] = make_float2(0.0f, 0.0f);
             if (row < kParamCount && inherited) {
-                pairs[k] = load_moments(previous, moment_index(parent, row));
+                const int64_t index = moment_index(parent, row);
+                if (Streaming) {
+                    const moment_pair q = load_moments(previous, index);
+                    pairs[k] = make_float2(q.x, q.y);
+                }
+                else {
+                    pairs[k] = *reinterpret_cast<const float2*>(previous + index);
+                }
             }
         }
 #pragma unroll
         for (int k = 0; k < kRemapRows; ++k) {
             const int row = base + k;
             if (row < kParamCount) {
-                store_moments(moments, moment_index(id, row), pairs[k].x, pairs[k].y);
+                const int64_t index = moment_index(id, row);
+                if (Streaming) {
+                    store_moments(moments, index, pairs[k].x, pairs[k].y);
+                }
+                else {
+                    *reinterpret_cast<float2*>(moments + index) = pairs[k];
+                }
             }
         }
     }
@@ -1044,8 +1062,10 @@ extern "C" int gsn_remap_history(gsn_context* context, const int* parent_ids, in
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_remap_history: null or aliased moment buffer");
     }
     StageScope scope(context, kStageDensity);
-    remap_history_kernel<<<grid_for(count, 256), 256, 0, context->stream>>>(parent_ids, previous_moments, moments,
-        previous_moments ? previous_count : 0, count);
+    const int inherited = previous_moments ? previous_count : 0;
+    const int64_t bytes = (static_cast<int64_t>(inherited) + count) * kParamCount * sizeof(moment_pair);
+    auto* kernel = bytes > kStreamedBytes ? remap_history_kernel<true> : remap_history_kernel<false>;
+    kernel<<<grid_for(count, 256), 256, 0, context->stream>>>(parent_ids, previous_moments, moments, inherited, count);
     return check_launch("remap_history_kernel");
 }
 
