@@ -55,10 +55,26 @@ __global__ __launch_bounds__(kEvalThreads) void quantized_error_kernel(const flo
         }
         done = fours * 4;
     }
-    for (int64_t i = done + thread; i < values; i += threads) {
-        const uint8_t q = one(image[i], static_cast<int>(target[i]));
-        if (quantized) {
-            quantized[i] = q;
+    // A value an access: several of a thread's loads in flight (5187x3361: 189 us one by one, 68 so).
+    constexpr int kBatch = Wide ? 1 : 8;
+    for (int64_t base = done + thread; base < values; base += kBatch * threads) {
+        float v[kBatch];
+        uint8_t t[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int64_t i = min(base + j * threads, values - 1);
+            v[j] = image[i];
+            t[j] = target[i];
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int64_t i = base + j * threads;
+            if (i < values) {
+                const uint8_t q = one(v[j], static_cast<int>(t[j]));
+                if (quantized) {
+                    quantized[i] = q;
+                }
+            }
         }
     }
 #pragma unroll
