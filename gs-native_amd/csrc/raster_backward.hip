@@ -650,7 +650,12 @@ int launch_splat_backward(gsn_context* context, const Camera& cam, int count, co
     // Four waves per tile while the tiles are few, one otherwise. Measured (us, four / two / one wave
     // per tile): 256 tiles 102 / 156 / 226, 1,024 tiles 110 / 161 / 236, 4,056 tiles 274 / 240 / 238,
     // 8,160 tiles 468 / 389 / 345; with one wave per tile and ten lane reads per splat the same images
-    // took 241, 241, 256 and 397. Stored form, 4,108 tiles: 259 / 233 / 204, before 236.
+    // took 241, 241, 256 and 397. Stored form, 4,108 tiles: 259 / 233 / 204, before 236. Over ten scenes a
+    // tile count, even and clustered, 60 to 1,500 records a tile, as shares of those times in the
+    // geometric mean [worst], four waves and one: 1,024 tiles .65 [.80], 1.00 [1.01]; 2,560 .75 [.96], .93
+    // [1.02]; 3,072 .79 [1.07], .92 [1.01]; 4,000 .89 [1.11], .91 [1.01]; 6,144 1.00 [1.17], .90 [.98]. Even
+    // lists would want the line at about 2,000 tiles, clustered ones past 6,000; the tile count does not
+    // tell them apart. Two waves were measured and are not launched.
     if (tiles <= 3072) {
         stored ? launch(raster_backward_kernel<1, true>, 4) : launch(raster_backward_kernel<1, false>, 4);
     }

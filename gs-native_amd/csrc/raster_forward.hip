@@ -233,9 +233,12 @@ int render_tiles(gsn_context* context, const gsn_camera* camera, const int* tile
 // issue, and bands that share a wave share its list and masks. Measured (us, one / two / four bands
 // per wave): 256 tiles 42 / 72 / 123, 1,024 tiles 54 / 84 / 131, 2,170 tiles 66 / 72 / 90, 4,056 tiles
 // 101 / 96 / 110, 8,160 tiles 175 / 158 / 162, 32,400 tiles 524 / 440 / 399; with one wave per tile
-// and nine lane reads per splat the same images took 142, 140, 131, 153, 211 and 570.
+// and nine lane reads per splat the same images took 142, 140, 131, 153, 211 and 570. Over ten scenes a
+// tile count, even and clustered, 60 to 1,500 records a tile, as shares of those times in the geometric
+// mean [worst]: 3,072 tiles .56 [.85] / .60 [.74] / .78 [.86], 8,160 .84 [1.67] / .71 [.91] / .74 [.89],
+// 9,600 .83 / .69 [.93] / .69 [.78], 12,288 .85 / .68 [1.04] / .66 [.76].
 int forward_bands(unsigned tiles) {
-    return tiles <= 3072 ? 1 : tiles <= 12288 ? 2 : 4;
+    return tiles <= 3072 ? 1 : tiles <= 9600 ? 2 : 4;
 }
 
 int launch_forward(gsn_context* context, const Camera& cam, const int* tile_gaussian_ids,

@@ -8,8 +8,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 CORNER = (61, 83)  # rows, columns: not multiples of the 16-pixel tile nor of the 4-row band
-# Tiles on either side of each boundary of the rules (3,072 and 12,288), and one row of tiles.
-CANVASES = [(61, 83), (768, 1024), (768, 1040), (1536, 2048), (1536, 2064), (16 * 3073, 16)]
+# Tiles on either side of each boundary of the rules (3,072 and 9,600), more, and one row of tiles.
+CANVASES = [(61, 83), (768, 1024), (768, 1040), (1536, 1600), (1536, 1616), (1536, 2048), (1536, 2064), (16 * 3073, 16)]
 
 
 def _draw(gsn, context, scenes, canvas, stored):
