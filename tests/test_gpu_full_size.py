@@ -2,8 +2,8 @@
 seeded 64-blob mixture, 1920x1080, SH degree 3 (the oracle's per-pixel restatement is too slow
 for this size, so these checks use invariants that hold at any size):
 
-- tile lists: the (tile << 32 | depth bits) keys are non-decreasing, tile offsets are exactly the
-  first index of each tile, every Gaussian has rectangle-area records, each record's tile lies in
+- tile lists: the (tile << 32 | depth bits) keys are non-decreasing, every tile's list is as long as
+  the number of rectangles on it, every Gaussian has rectangle-area records, each record's tile lies in
   its Gaussian's rectangle, and records with equal keys keep Gaussian-id order (the reference's
   stable order);
 - the gradient pass is deterministic (two runs agree bit for bit) and the fused gradient + Adam
@@ -55,6 +55,12 @@ def test_tile_lists_invariants_at_full_size(gsn, context, full_scene):
     areas = (rects[:, 2] - rects[:, 0]).astype(np.int64) * (rects[:, 3] - rects[:, 1])
     np.testing.assert_array_equal(counts[visible], areas[visible])
     assert counts.sum() == r
+    # Rectangles on each tile: a difference array over the grid, summed along both axes.
+    corners = np.zeros((cam.tile_count_y + 1, cam.tile_count_x + 1), np.int64)
+    for x, y, sign in ((0, 1, 1), (2, 1, -1), (0, 3, -1), (2, 3, 1)):
+        np.add.at(corners, (rects[visible, y], rects[visible, x]), sign)
+    on_tile = corners.cumsum(axis=0).cumsum(axis=1)[:-1, :-1].ravel()
+    np.testing.assert_array_equal(offsets, np.concatenate([[0], np.cumsum(on_tile)]))
     tx, ty = tiles % cam.tile_count_x, tiles // cam.tile_count_x
     rect = rects[ids]
     assert np.all((tx >= rect[:, 0]) & (tx < rect[:, 2]) & (ty >= rect[:, 1]) & (ty < rect[:, 3]))

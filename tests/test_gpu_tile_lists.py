@@ -1,6 +1,7 @@
 """gsn_build_tile_lists against a NumPy stable sort by (tile, depth, id), over grids and counts on
 either side of the edges of its decomposition: 32x32-tile parts, 8x8-tile regions,
-64-entry queues, 4,096-entry lists and chunks of 256 to 8,192 entries. Integers: equal."""
+64-entry queues, 4,096-entry lists and chunks of 256 to 8,192 entries, all of which count and
+write (at least a quarter record per entry and part). Integers: equal."""
 import ctypes
 
 import numpy as np
@@ -15,7 +16,8 @@ CASES = [
     (120, 68, 3000, 120),  # rectangles up to the whole screen
     (1, 300, 700, 4), (300, 1, 700, 4),  # strips
     (512, 511, 12_000, 9), (513, 130, 40_000, 30),  # many parts, ragged last ones
-    (40, 33, 1_500_000, 2),  # the longest chunks
+    (40, 33, 1_500_000, 2),  # chunks of 4,096 entries
+    (120, 68, 750_000, 3),  # chunks of 8,192 entries, two lists each
     (65_535, 1, 500, 4), (1, 65_535, 500, 4),  # the largest
 ]
 
