@@ -330,12 +330,12 @@ __device__ __forceinline__ void write_statistics(const Camera& cam, const float 
 // all 64 lanes of the wave call it together. slots: the wave's LDS staging area,
 // kChunks * 64 * 3 float4.
 // Each Gaussian owns the contiguous run of partial records of its tile rectangle, so a wave's 64
-// Gaussians own one contiguous run. The backward wrote a partial only for the records its tile
-// reached before every pixel was done, and stamped those records' flag bytes with this step's
-// epoch (at 1080p with a converged scene about 4% of the records). The wave walks its run
-// kChunks x 64 records at a time, one record per lane and chunk: the flag bytes are read
-// together, the stamped partials are loaded (coalesced, neighbouring lanes hold neighbouring
-// records) into the wave's LDS slots, and each lane then adds the stamped records of its own
+// Gaussians own one contiguous run. The backward stamped the flag bytes of the records its tile
+// reached before every pixel was done with this step's epoch (at 1080p with a converged scene about
+// 4% of the records), and wrote a partial, marked by kFlagPartial, for those that a pixel blended.
+// The wave walks its run kChunks x 64 records at a time, one record per lane and chunk: the flag bytes
+// are read together, the partials are loaded (coalesced, neighbouring lanes hold neighbouring
+// records) into the wave's LDS slots, and each lane then adds the partials of its own
 // Gaussian from LDS in record order; a Gaussian owning kWideOwner or more of a chunk's stamped
 // records instead adds the chunk's wave-wide sum of them. Every order is fixed, so results are
 // identical run to run. Work per wave

@@ -172,7 +172,7 @@ int check_launch(const char* kernel);
 // Returns a device buffer of at least `bytes` for `slot`, growing it if needed (no copy).
 void* scratch(gsn_context* context, ScratchSlot slot, size_t bytes);
 
-// Image metrics (ssim.hip): partial sums per 32x16 block and channel into block_sums
+// Image metrics (ssim.hip): partial sums per 32x32 block and channel into block_sums
 // (image_metric_blocks(width, height) x 3 doubles), then a fixed-order finish into out[4] (device).
 int64_t image_metric_blocks(int width, int height);
 int launch_image_metrics(gsn_context* context, int width, int height, const float* image, const uint8_t* target,
@@ -238,10 +238,10 @@ struct StoredState {
 };
 
 // Tile rasteriser backward writing per-record partials (raster_backward.hip): the recompute form
-// when stored is null, else the back-to-front stored-state form. Only the records a tile reaches
-// before all its pixels are done get a partial; for each of them the backward also stores the
-// step's epoch into record_flags[slot] (*flags, *epoch are returned), so the per-Gaussian pass
-// reads exactly the partials written in this step.
+// when stored is null, else the back-to-front stored-state form. The records a tile reaches before
+// all its pixels are done get the step's epoch in record_flags[slot] (*flags, *epoch are returned);
+// those that some pixel blended also get kFlagPartial there and a partial, so the per-Gaussian
+// pass reads exactly the partials written in this step.
 // Makes these buffers the context's last projection (project.hip): the tile-list build, the depth
 // order queued by the record scan and the backward prefetch refer to it.
 int record_projection(gsn_context* context, int count, float* means, float* conic_opacities, float* colors,

@@ -1,7 +1,8 @@
 // Stable LSD radix sort of (uint32 key, uint32 value) pairs for wave64 / gfx950.
 //
 // Each pass (<= 8 digit bits) runs three kernels over 4096-element tiles:
-//   1. radix_histogram: per-tile digit histogram in LDS, written bin-major [bin][tile].
+//   1. radix_histogram: per-tile digit histogram in LDS, written bin-major [bin][tile], of few tiles
+//      (kFusedTiles) tile-major [tile][256].
 //   2. radix_digit_scan: one workgroup per digit scans its row of the table in place (the
 //      digit's start inside every tile's share) and writes the row total. Few tiles do without: the
 //      scatter's workgroups add up the counts themselves.
@@ -283,9 +284,6 @@ int* radix_histogram_buffer(gsn_context* context, int64_t n) {
         scratch(context, kSlotSortHistogram, (static_cast<size_t>(tiles) + 1) * 256 * sizeof(int)));
 }
 
-// Digit widths: the narrower digits come first (13 tile bits: 6 then 7). The first pass of the
-// tile sort reads the records in emission order, where neighbouring records share tiles; fewer
-// bins there measured slightly faster (tile sort 0.298 -> 0.291 ms at 30M records).
 // Up to this many tiles the scatter forms the digits' starts itself.
 static constexpr int kFusedTiles = 128;
 
@@ -293,6 +291,10 @@ bool radix_table_by_tile(int64_t n) {
     return (n + kSortTile - 1) / kSortTile <= kFusedTiles;
 }
 
+// Digit widths: the narrower digits come first (13 tile bits: 6 then 7). The first pass of the sort
+// of tile records reads them in emission order, where neighbouring records share tiles; fewer
+// bins there measured slightly faster (0.298 -> 0.291 ms at 30M records). 30 and 32 bits: 7, 7, 8, 8 and
+// four times 8.
 int radix_first_digit_bits(int bits) {
     bits = bits < 1 ? 1 : (bits > 32 ? 32 : bits);
     int passes = (bits + 7) / 8;

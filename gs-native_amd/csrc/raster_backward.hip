@@ -197,6 +197,7 @@ __global__ __launch_bounds__(64 * (4 / Bands)) void raster_backward_kernel(const
     const float* __restrict__ final_transmittance, const int* __restrict__ last_contributor,
     const float* __restrict__ image_gradients, float bg_r, float bg_g, float bg_b, float* __restrict__ partials,
     uint8_t* __restrict__ record_flags, uint8_t epoch, int record_count) {
+    static_assert(Bands == 1 || Bands == 4, "the forms that are launched");
     constexpr int kWaves = 4 / Bands;
     constexpr bool kIfs = Stored && Bands > 1, kSelects = Stored && Bands == 1;
     // A wave's records of the batch, in order: centre x, y, conic a, b | conic c, opacity, red, green |

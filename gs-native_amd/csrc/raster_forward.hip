@@ -206,7 +206,7 @@ int render_tiles(gsn_context* context, const gsn_camera* camera, const int* tile
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_render_tiles: invalid arguments");
     }
     int64_t tiles = static_cast<int64_t>(camera->tile_count_x) * camera->tile_count_y;
-    if (tiles >= 0x1fffffff) {
+    if (tiles >= 0x7fffffff) {
         return fail(GSN_ERROR_INVALID_ARGUMENT, "gsn_render_tiles: too many tiles");
     }
     Camera cam;

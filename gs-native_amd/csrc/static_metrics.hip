@@ -59,7 +59,7 @@ extern "C" int gsn_image_metrics_static(gsn_context* context, int width, int hei
     if (blocks > kStaticMetricBlocks) {
         return fail(GSN_ERROR_CAPACITY,
             "gsn_image_metrics_static: a %dx%d image needs %lld partial-sum blocks, above the static maximum of %lld "
-            "(about 22 million pixels)",
+            "(about 44 million pixels)",
             width, height, static_cast<long long>(blocks), static_cast<long long>(kStaticMetricBlocks));
     }
     if (!context->static_scratch) {

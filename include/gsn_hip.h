@@ -133,7 +133,7 @@ int gsn_selftest_wave_sum12(gsn_context* context, const float* input, float* out
 int gsn_selftest_band_mask(gsn_context* context, const float* splats, const int* origins, int count, int* masks);
 
 /* Diagnostic: the library's stable radix sort of (uint32 key, uint32 value) pairs by key bits
- * [0, bits) (1 <= bits <= 32), as the depth order, the tile lists and the KNN use it: keys and
+ * [0, bits) (1 <= bits <= 32), as the depth order, the tile records and the KNN use it: keys and
  * values (device, count each) are consumed, the sorted pairs go to keys_out / values_out (device,
  * distinct from the inputs). Its counterpart in the reference is the CUB
  * DeviceRadixSort::SortPairs call of renderer.cu:546-563. */
@@ -212,8 +212,8 @@ int gsn_image_quantized_error(gsn_context* context, int width, int height, const
 /* Allocation-free gsn_image_metrics: no counterpart in the reference. For callers that cannot
  * allocate device memory (code under HIP graph capture, evaluation loops that must not call
  * hipMalloc). Same kernels and results (bit for bit) as gsn_image_metrics, but the per-block
- * partial sums live in a file-scope device array of 3 MiB per device (131,072 blocks of 32x16
- * pixels per channel: images up to about 22 million pixels; larger ones return
+ * partial sums live in a file-scope device array of 3 MiB per device (131,072 blocks of 32x32
+ * pixels of a channel: images up to about 44 million pixels; larger ones return
  * GSN_ERROR_CAPACITY), and the four results are written to device_out (4 doubles of device
  * memory) without synchronising the stream. Calls that overlap on one device share that array
  * and race; calls on one context's stream are ordered and safe. */

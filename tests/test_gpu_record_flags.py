@@ -1,6 +1,6 @@
-"""The backward stamps every record it reaches with a per-step epoch byte (1..255) that the
+"""The backward stamps every record it reaches with a per-step epoch (1..127; bit 7 says that the record has a partial) that the
 per-Gaussian pass compares against; the flag buffer is cleared when it is allocated and when the
-epoch wraps. These tests drive one context through more than 255 gradient steps, alternating
+epoch wraps. These tests drive one context through more than twice 127 gradient steps, alternating
 two projections with different record counts, and require every step to reproduce that
 projection's first result bit for bit: a stale stamp that matched the current epoch would add a
 stale partial, and a missing stamp would drop one.
@@ -12,7 +12,7 @@ from helpers import config0_camera
 
 pytestmark = pytest.mark.gpu
 
-STEPS = 300  # past one epoch wrap (255 steps)
+STEPS = 300  # past two epoch wraps (127 steps each)
 
 
 def _projection(gsn, context, params, cam, sh_degree):

@@ -176,10 +176,9 @@ def test_tile_lists_rebuilt_without_queued_depth_order(gsn, context, scenes):
 
 def test_tile_lists_with_empty_rectangles_between_records(gsn, context):
     """Inputs the projection never writes: 5,000 Gaussians marked visible by their record offsets
-    but with empty tile rectangles, between two runs of two-record Gaussians. The first
-    4096-record block then has more owners than positions, and the emission finds each record's
-    owner by binary search. The lists must equal a stable sort by (tile, depth) of the records in
-    depth order, which here is id order (depths increase with the id)."""
+    but with empty tile rectangles, between two runs of two-record Gaussians. The lists must equal a
+    stable sort by (tile, depth) of the records in depth order, which here is id order (depths
+    increase with the id)."""
     normal_before, empty, normal_after = 2000, 5000, 5000
     count = normal_before + empty + normal_after
     f = 600.0
