@@ -15,10 +15,10 @@
 // one record per tile, and equal depth bits keep id order in both).
 // Why not a sort: a record then costs 4 bytes written, once, instead of about 48 bytes of traffic
 // through the emission of (tile, id) pairs, two radix passes over them and the search for the tiles'
-// ranges. What bounds it now: the gather of step 2 (a random line per Gaussian) and, in step 5, vector
-// instructions. Emission to ranges with the sort and so: 10K Gaussians at 256x256 45 and 25 us, 200K
-// at 979x546 88 and 73, 500K at 1248x832 160 and 113, 3M at 1920x1080 660 and 494, 2M at 3840x2160
-// 2,100 and 640.
+// ranges. What bounds it now: the gather of step 2 (a random line per Gaussian) and step 5 (see
+// tile_write_kernel). Emission to ranges with the sort and so: 10K Gaussians at 256x256 45 and 25 us, 200K
+// at 979x546 88 and 71, 500K at 1248x832 160 and 114, 3M at 1920x1080 660 and 467, 2M at 3840x2160
+// 2,100 and 605.
 // Lists with few records per entry and part are sorted after all (lists_by_records).
 #include "raster_common.h"
 
@@ -474,14 +474,15 @@ __global__ __launch_bounds__(1024) void tile_offsets_kernel(int* totals, const i
 // meet the region wait in a queue until a full wave of them is there. Every tile's set of queued
 // entries is a lane mask, the AND of a row's and a column's, and the places of the region's tiles,
 // one per lane, advance by its population count.
-// What bounds it: instructions, half of them the seven per tile and queue (store_row), a quarter the
-// walk of the list and a quarter the gathering (3M Gaussians at 1920x1080: 195, 85 and 92 us of 385 with
-// four-byte corners in the list and the compiler's selects, 342 in all so; without the stores
-// themselves 371); and a workgroup's busiest region, since splats of one depth crowd together. Eight
-// waves a SIMD let two workgroups fit on a CU. Dealing out the rows
-// of the regions evenly, with a list per region, took more instructions and more time (732 against
-// 501 us, 3M Gaussians at 1920x1080, both before the stores were written out); counters in LDS and a
-// scattered store per record 826 us; ids staged per tile in LDS 1,032 us (three waves on a SIMD).
+// What bounds it: the length of a wave's chains (list, queue, masks, stores) and the barriers around
+// a workgroup's list, which wait for its busiest region, since splats of one depth crowd together: at
+// 3M Gaussians, 1920x1080, its 319 us fill 0.36 of the VALU's issue slots, and a wave waits half its
+// time. Half of it are the seven instructions per tile and queue (store_row), a quarter the walk of the
+// list and a quarter the gathering (195, 85 and 92 us of 385 with four-byte corners in the list and the
+// compiler's selects; without the stores themselves 371). Eight waves a SIMD let two workgroups fit on
+// a CU. Dealing out the rows of the regions evenly, with a list per region, took more time (732 against
+// 501 us, both before the stores were written out); counters in LDS and a scattered store per record
+// 826 us; ids staged per tile in LDS 1,032 us (three waves on a SIMD).
 constexpr int kListEntries = 4096;
 constexpr int kRegionSide = 8;
 constexpr int kRegions = kPartTiles / 64;  // waves of a workgroup
