@@ -226,14 +226,14 @@ constexpr int kCornerStride = kPartSide + 1;
 __device__ __forceinline__ int count_entries(const uint2* __restrict__ rects, const PartTask& task,
     int (&s_corner)[kCornerStride * kCornerStride]) {
     constexpr int kStride = kCornerStride;
-    for (int i = threadIdx.x; i < kStride * kStride; i += kPartThreads) {
-        s_corner[i] = 0;
-    }
-    __syncthreads();
     uint2 next = make_uint2(0u, 0u);
     if (task.begin + threadIdx.x < task.end) {
         next = rects[task.begin + threadIdx.x];
     }
+    for (int i = threadIdx.x; i < kStride * kStride; i += kPartThreads) {
+        s_corner[i] = 0;
+    }
+    __syncthreads();
     for (int64_t k = task.begin + threadIdx.x; k < task.end; k += kPartThreads) {
         const uint2 rect = next;
         if (k + kPartThreads < task.end) {
