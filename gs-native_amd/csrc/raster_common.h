@@ -95,9 +95,12 @@ __device__ __forceinline__ int band_mask(float mx, float my, float4 conic, int x
     float det = a * c - b * b;
     // det, a and c inside the range where their reciprocals and they themselves are normal numbers: the
     // hardware's reciprocal takes a subnormal operand for zero and gives zero for a subnormal result.
-    constexpr float kSmallest = 0x1p-125f, kLargest = 0x1p125f;
-    if (!(det >= kSmallest) || !(fminf(a, c) >= kSmallest) || !(fmaxf(det, fmaxf(a, c)) <= kLargest) ||
-        !isfinite(mx) || !isfinite(my)) {
+    // (Bits of positive floats are ordered like their values: one comparison for the three, which also
+    // turns negative values, infinities and NaN away.)
+    constexpr uint32_t kSmallest = (127u - 125u) << 23, kLargest = (127u + 125u) << 23;  // 2^-125, 2^125
+    const uint32_t beyond = max(max(__float_as_uint(a) - kSmallest, __float_as_uint(c) - kSmallest),
+        __float_as_uint(det) - kSmallest);
+    if (beyond > kLargest - kSmallest || !isfinite(mx) || !isfinite(my)) {
         return kAll;
     }
     float tau = __logf(255.0f * o) + 0.25f;
